@@ -304,6 +304,7 @@ struct bnr_ctx {
   // launch at or above this many workgroups
   int gemv_norm_min_wgs = 256;
   int pf_pair = -1;               // paired 16-query launches: -1 planner (4 q heads per kv head), 0 never, 1 where possible
+  int pf_split = -1;              // fp16-pair prefill: -1 by shape unless another launch is forced, 0 never, 1 wherever it fits
   std::vector<PrefillPlanEntry> pf_plans;  // recent (shape -> key tiles per chunk) plans
 };
 
@@ -930,6 +931,7 @@ extern "C" int bnr_create(int device_id, bnr_ctx **out) {
   if (const char *v = std::getenv("BNR_PREFILL_BALANCED")) c->pf_balanced = std::min(1, std::max(-1, atoi(v)));
   if (const char *v = std::getenv("BNR_GEMV_NORM_MIN_WGS")) c->gemv_norm_min_wgs = std::max(1, atoi(v));
   if (const char *v = std::getenv("BNR_PREFILL_PAIR")) c->pf_pair = std::min(1, std::max(-1, atoi(v)));
+  if (const char *v = std::getenv("BNR_PREFILL_SPLIT")) c->pf_split = std::min(1, std::max(-1, atoi(v)));
   if (const char *v = std::getenv("BNR_PREFILL_MODE")) {
     const int m = atoi(v);
     if (m >= kPrefillGrid && m <= kPrefillAuto) c->pf_mode = m;
@@ -1364,9 +1366,9 @@ int check_rows(size_t last_pos, size_t cap) {
 
 bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
-int launch_rope_append_dev(bnr_ctx *c, float *q, float *k, const float *v, size_t n_tokens,
-                           size_t start_pos, size_t n_heads, size_t n_kv, size_t head_dim,
-                           float *k_cache, float *v_cache, size_t cap, hipStream_t s) {
+RopeAppendArgs rope_append_args(const bnr_ctx *c, float *q, float *k, const float *v,
+                                size_t n_tokens, size_t start_pos, size_t n_heads, size_t n_kv,
+                                size_t head_dim, float *k_cache, float *v_cache, size_t cap) {
   RopeAppendArgs a{};
   a.q = q;
   a.k = k;
@@ -1381,6 +1383,14 @@ int launch_rope_append_dev(bnr_ctx *c, float *q, float *k, const float *v, size_
   a.k_cache = k_cache;
   a.v_cache = v_cache;
   a.kv_stride = (long long)(cap * head_dim);
+  return a;
+}
+
+int launch_rope_append_dev(bnr_ctx *c, float *q, float *k, const float *v, size_t n_tokens,
+                           size_t start_pos, size_t n_heads, size_t n_kv, size_t head_dim,
+                           float *k_cache, float *v_cache, size_t cap, hipStream_t s) {
+  const RopeAppendArgs a = rope_append_args(c, q, k, v, n_tokens, start_pos, n_heads, n_kv,
+                                            head_dim, k_cache, v_cache, cap);
   HIP_TRY(launch_rope_append(a, s), "rope/append launch");
   return BNR_OK;
 }
@@ -1723,6 +1733,101 @@ bool prefill_streamk_shape(const bnr_ctx *c, size_t n_tokens, size_t start_pos) 
           (c->pf_mode == kPrefillAuto && start_pos >= n_tokens && n_tokens > 512));
 }
 
+// Floats of partial states and tickets a context keeps for prefills on a
+// cache of `cap` rows, whatever launch needs `min_items` (kv head, item) pairs
+// of them: sized for every launch on that cache, so that later calls on it
+// (also under HIP graph capture) never allocate.
+int ensure_prefill_ws(bnr_ctx *c, long long cap, long long n_qtiles, int n_kv, int group,
+                      long long budget_items, long long min_items) {
+  const int per_cu = group >= 8 ? 1 : 2;  // resident workgroups per CU (registers, LDS)
+  const long long T = (cap + 31) / 32;
+  const long long items = std::max({budget_items, min_items, 2LL * c->n_cu * per_cu});
+  int st = ensure_buf(&c->pf_ws, &c->pf_ws_floats, (size_t)items * group * 66 * 64,
+                      "prefill workspace alloc");
+  if (st) return st;
+  // tickets: one per (kv head, query tile, 16-query half)
+  return ensure_zeroed(&c->pf_counters, &c->n_pf_counters,
+                       (size_t)n_kv * std::max<long long>(T, n_qtiles) * 2 * kCounterStride);
+}
+
+// The part of that workspace a split launch's K/V tiles and their words take
+// (floats, rounded up to 1 KB), at its start; the states follow.
+long long split_tile_floats(long long cap, int n_kv) {
+  const long long tiles = n_kv * ((cap + 31) / 32);
+  return (tiles * kSplitTileFloats + 2 * tiles + 255) & ~255LL;
+}
+
+// States per kv head a split launch can keep beside its tiles in the
+// workspace every prefill on a cache of `cap` rows reserves anyway.
+long long split_slots(const bnr_ctx *c, long long cap, int n_kv, int group) {
+  const int per_cu = group >= 8 ? 1 : 2;
+  const long long items = std::max(prefill_item_budget(cap, n_kv), 2LL * c->n_cu * per_cu);
+  return (items * group * 66 * 64 - split_tile_floats(cap, n_kv)) /
+         ((long long)split_waves(group) * 66 * 64 * n_kv);
+}
+
+// Whether a prefill of a tiled shape runs as a split launch: nothing else is
+// forced, and (prefill_split_plan, which fills in its runs) its tiles leave at
+// least half of the workspace to the states, and the launch is large enough to
+// pay for the tiles and the longer start: at least kSplitTokens new tokens, or kSplitRows query
+// rows times keys (MI355X, 20/5 heads, RoPE + append + attention in us, fp32
+// launches against split: 256 tokens 18.5 / 22.7, 512 29.9 / 28.6, 1024 62 /
+// 42, 2048 200 / 94, 4000 680 / 267; 64 after 2000 30 / 37, 128 after 3900 59 /
+// 56, 333 after 1207 54 / 43, 512 after 1536 91 / 51).
+constexpr size_t kSplitTokens = 512, kSplitRows = 400000;
+bool prefill_split_shape(const bnr_ctx *c, size_t n_tokens, size_t start_pos) {
+  if (c->pf_split >= 0) return c->pf_split != 0;
+  const bool forced = c->pf_mode != kPrefillAuto || c->pf_chunk_tiles > 0 || c->pf_q16 >= 0 ||
+                      c->pf_balanced >= 0 || c->pf_pair >= 0;
+  return !forced &&
+         (n_tokens >= kSplitTokens || n_tokens * (start_pos + n_tokens / 2) >= kSplitRows);
+}
+bool prefill_split_plan(const bnr_ctx *c, size_t n_tokens, size_t start_pos, size_t cap,
+                        size_t n_heads, size_t n_kv, PrefillRunsArgs &a) {
+  const int group = (int)(n_heads / n_kv);
+  const long long slots = split_slots(c, (long long)cap, (int)n_kv, group);
+  if (slots * split_waves(group) * 66 * 64 * (long long)n_kv < split_tile_floats((long long)cap, (int)n_kv))
+    return false;
+  a.n_tokens = (int)n_tokens;
+  a.start_pos = (int)start_pos;
+  a.n_heads = (int)n_heads;
+  a.n_kv = (int)n_kv;
+  return plan_prefill_runs(a, group, c->n_cu, slots);
+}
+
+// Prefill attention as a split launch (a planned by prefill_split_plan),
+// c->mu held: K/V tiles as fp16 pairs, then attention over them.  rope: q, k
+// and v are raw and the first launch rotates and appends them too (16-byte
+// aligned); otherwise the cache holds every row.
+int prefill_split_locked(bnr_ctx *c, PrefillRunsArgs &pa, const RopeAppendArgs &rope_args, bool rope,
+                         float *out, long long cap, hipStream_t s) {
+  const int n_kv = pa.n_kv, group = pa.n_heads / n_kv;
+  const int st = ensure_prefill_ws(c, cap, pa.n_units, n_kv, group, prefill_item_budget(cap, n_kv), 0);
+  if (st) return st;
+  PrefillSplitArgs sa{};
+  sa.rope = rope_args;
+  if (!rope) sa.rope.cos_tab = nullptr;
+  sa.n_tiles = (pa.start_pos + pa.n_tokens + 31) / 32;
+  sa.tiles_per_head = (cap + 31) / 32;
+  sa.tiles = c->pf_ws;
+  sa.info = reinterpret_cast<int2 *>(c->pf_ws + n_kv * sa.tiles_per_head * kSplitTileFloats);
+  HIP_TRY(launch_prefill_split_kv(sa, s), "prefill tiles launch");
+  pa.q = rope_args.q;
+  pa.k_cache = rope_args.k_cache;
+  pa.v_cache = rope_args.v_cache;
+  pa.kv_stride = rope_args.kv_stride;
+  pa.out = out;
+  pa.scale_log2 = 1.4426950408889634f / sqrtf((float)kHeadDim);
+  pa.timeline = c->timeline;
+  pa.tiles = sa.tiles;
+  pa.info = sa.info;
+  pa.tiles_per_head = sa.tiles_per_head;
+  pa.ws = c->pf_ws + split_tile_floats(cap, n_kv);
+  pa.counters = c->pf_counters;
+  HIP_TRY(launch_prefill_split(pa, group, s), "prefill launch");
+  return set_ok();
+}
+
 // Prefill attention with c->mu held.
 int prefill_attention_locked(bnr_ctx *c, const float *q, const float *k_cache,
                              const float *v_cache, size_t cap, float *out, size_t n_tokens,
@@ -1733,6 +1838,16 @@ int prefill_attention_locked(bnr_ctx *c, const float *q, const float *k_cache,
   const long long kv_stride = (long long)(cap * head_dim);
   const int group = (int)(n_heads / n_kv_heads);
   if (prefill_tiled(n_tokens, start_pos, n_heads, n_kv_heads, head_dim, q, k_cache, v_cache, out)) {
+    if (prefill_split_shape(c, n_tokens, start_pos)) {
+      PrefillRunsArgs ra{};
+      if (prefill_split_plan(c, n_tokens, start_pos, cap, n_heads, n_kv_heads, ra))
+        return prefill_split_locked(
+            c, ra,
+            rope_append_args(c, const_cast<float *>(q), nullptr, nullptr, n_tokens, start_pos,
+                             n_heads, n_kv_heads, head_dim, const_cast<float *>(k_cache),
+                             const_cast<float *>(v_cache), cap),
+            false, out, (long long)cap, s);
+    }
     PrefillArgs pa{};
     pa.q = q;
     pa.k_cache = k_cache;
@@ -1780,25 +1895,16 @@ int prefill_attention_locked(bnr_ctx *c, const float *q, const float *k_cache,
     pa.n_items = plan.n_items;
     prefill_order(pa);
     {
-      // Partial states and tickets, sized -- whatever this launch needs --
-      // for every launch on a cache of `cap` rows, so that later calls on it
-      // (also under HIP graph capture) never allocate: stream-K launches keep
-      // two states per resident workgroup; a planned chunk size keeps to
-      // prefill_item_budget (kv head, item) pairs; a forced one (tuning) to
-      // T = cap/32 query tiles of at most ceil(T / chunk) chunks each.
+      // stream-K launches keep two states per resident workgroup; a planned
+      // chunk size keeps to prefill_item_budget (kv head, item) pairs; a forced
+      // one (tuning) to T = cap/32 query tiles of at most ceil(T / chunk)
+      // chunks each.
       const long long T = ((long long)cap + 31) / 32;
-      long long items = c->pf_chunk_tiles > 0
-                            ? (long long)n_kv_heads * T * ((T + pa.chunk_tiles - 1) / pa.chunk_tiles)
-                            : prefill_item_budget((long long)cap, (int)n_kv_heads);
-      if (plan.split) items = std::max<long long>(items, (long long)n_kv_heads * plan.n_items);
-      items = std::max<long long>(items, 2LL * c->n_cu * per_cu);
-      st = ensure_buf(&c->pf_ws, &c->pf_ws_floats, (size_t)items * group * 66 * 64,
-                      "prefill workspace alloc");
-      if (st) return st;
-      // tickets: one per (kv head, query tile, 16-query half)
-      st = ensure_zeroed(&c->pf_counters, &c->n_pf_counters,
-                         (size_t)n_kv_heads * std::max<long long>(T, pa.n_qtiles) * 2 *
-                             kCounterStride);
+      const long long items = c->pf_chunk_tiles > 0
+                                  ? (long long)n_kv_heads * T * ((T + pa.chunk_tiles - 1) / pa.chunk_tiles)
+                                  : prefill_item_budget((long long)cap, (int)n_kv_heads);
+      st = ensure_prefill_ws(c, (long long)cap, pa.n_qtiles, (int)n_kv_heads, group, items,
+                             plan.split ? (long long)n_kv_heads * plan.n_items : 0);
       if (st) return st;
     }
     if (streamk) {
@@ -1898,6 +2004,17 @@ extern "C" int bnr_dev_prefill(bnr_ctx *c, float *q, float *k, const float *v, s
   hipStream_t s = (hipStream_t)stream;
   st = ensure_table(c, std::max(start_pos + n_tokens, cap) - 1, head_dim, theta);
   if (st) return st;
+  if (prefill_split_shape(c, n_tokens, start_pos) && aligned16(k) && aligned16(v) &&
+      prefill_tiled(n_tokens, start_pos, n_heads, n_kv_heads, head_dim, q, k_cache, v_cache, out)) {
+    PrefillRunsArgs ra{};
+    if (prefill_split_plan(c, n_tokens, start_pos, cap, n_heads, n_kv_heads, ra)) {
+      st = prefill_split_locked(c, ra,
+                                rope_append_args(c, q, k, v, n_tokens, start_pos, n_heads,
+                                                 n_kv_heads, head_dim, k_cache, v_cache, cap),
+                                true, out, (long long)cap, s);
+      return st ? st : set_ok();
+    }
+  }
   st = launch_rope_append_dev(c, q, k, v, n_tokens, start_pos, n_heads, n_kv_heads, head_dim,
                               k_cache, v_cache, cap, s);
   if (st) return st;

@@ -139,6 +139,18 @@ __device__ __forceinline__ void st4_agent(__amdgpu_buffer_rsrc_t r, int off, flo
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned, x),
                                          r, off, 0, 16);
 }
+// ... with a uniform part `soff` of the offset in a scalar register.
+__device__ __forceinline__ void st4_agent(__amdgpu_buffer_rsrc_t r, int off, int soff, float4 v) {
+  typedef float f4v __attribute__((ext_vector_type(4)));
+  const f4v x = {v.x, v.y, v.z, v.w};
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned, x),
+                                         r, off, soff, 16);
+}
+__device__ __forceinline__ float4 ld4_agent(__amdgpu_buffer_rsrc_t r, int off, int soff) {
+  typedef float f4v __attribute__((ext_vector_type(4)));
+  const f4v v = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 16));
+  return make_float4(v.x, v.y, v.z, v.w);
+}
 __device__ __forceinline__ void st2_agent(__amdgpu_buffer_rsrc_t r, int off, float a, float b) {
   typedef float f2v __attribute__((ext_vector_type(2)));
   const f2v x = {a, b};

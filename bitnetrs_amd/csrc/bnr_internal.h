@@ -526,6 +526,61 @@ __host__ __device__ inline SkSeg sk_seg(const PrefillArgs &a, long long u, long 
 }
 
 hipError_t launch_prefill(const PrefillArgs &a, int group, int persistent_wgs, hipStream_t s);
+
+// A 32-key K/V tile of one kv head as fp16 pairs: 16 KB of K operands, 16 KB
+// of V operands (prefill_split_kv_kernel has the order).
+constexpr int kSplitTileFloats = 2 * 32 * kHeadDim;
+// K/V tiles of cache rows 0 .. start_pos + n_tokens - 1 for a split prefill.
+// With rope.cos_tab the launch also rotates rope.q and rope.k, and appends k
+// and v, exactly as launch_rope_append; otherwise every row is read from the
+// cache and q, k and v are not used.
+struct PrefillSplitArgs {
+  RopeAppendArgs rope;
+  float *tiles;  // [n_kv][tiles_per_head][kSplitTileFloats]
+  int2 *info;    // [n_kv][tiles_per_head]: words of the K and the V part
+  int n_tiles;   // ceil((start_pos + n_tokens) / 32)
+  long long tiles_per_head;
+};
+hipError_t launch_prefill_split_kv(const PrefillSplitArgs &p, hipStream_t s);
+
+// Split prefill attention (prefill_split_kernel).  A workgroup is W waves
+// (split_waves): the G query heads of one kv head x W / G blocks of 32 queries,
+// a query unit of 32 W / G queries whose key tiles they share.  Unit u has
+// nk(u) = min(start_pos + (u + 1) 32 W / G, start_pos + n_tokens) / 32, rounded
+// up, key tiles; the units' tiles in order are one line per kv head, cut into
+// n_runs runs of about equal cost.  A workgroup takes one run; the pieces of a
+// unit that spans several runs leave their states in slots base .. base +
+// nch - 1 of the kv head, and the last to finish merges them.
+constexpr int split_waves(int group) { return group > 4 ? 8 : 4; }
+constexpr int split_unit(int group) { return 32 * split_waves(group) / group; }
+constexpr int kMaxPrefillRuns = 256;
+struct PrefillRunsArgs {
+  const float *q;                  // [n_tokens][n_heads][128], rotated
+  const float *k_cache, *v_cache;  // [n_kv][cap][128] (marked tiles)
+  long long kv_stride;
+  float *out;                      // [n_tokens][n_heads][128]
+  int n_tokens, start_pos, n_heads, n_kv;
+  float scale_log2;                // log2(e) / sqrt(128)
+  const float *tiles;              // PrefillSplitArgs
+  const int2 *info;
+  long long tiles_per_head;
+  float *ws;                       // states: [n_kv][n_slots][W][66][64]
+  unsigned *counters;              // [n_kv][n_units] x kCounterStride, zero between launches
+  int n_units, n_slots, n_runs;
+  int grid;                        // workgroups: n_kv * n_runs rounded up to a multiple of 16
+  unsigned long long *timeline;    // measurement builds: PfStamp records by workgroup
+  // Run r: first unit | its first tile << 16; tiles | pieces of the first
+  // unit << 16 | this piece's number << 24; the first unit's slot base | the
+  // last unit's << 10 | pieces of the last unit << 20 (the run holds its
+  // first piece).  Units between the two are whole.
+  unsigned run[kMaxPrefillRuns][3];
+};
+static_assert(sizeof(PrefillRunsArgs) <= 4096, "PrefillRunsArgs exceeds the kernel argument limit");
+// Fills n_units, n_slots, n_runs, grid and run[] from n_tokens, start_pos and
+// n_kv for workgroups of `group` heads on n_cu CUs, with at most max_slots
+// states per kv head.  False when the shape does not fit the words.
+bool plan_prefill_runs(PrefillRunsArgs &a, int group, int n_cu, long long max_slots);
+hipError_t launch_prefill_split(const PrefillRunsArgs &a, int group, hipStream_t s);
 // Stream-K prefill over `wgs` workgroups (a.sk_units, a.sk_per_head set by
 // prefill_streamk_units).
 hipError_t launch_prefill_streamk(const PrefillArgs &a, int group, int wgs, hipStream_t s);

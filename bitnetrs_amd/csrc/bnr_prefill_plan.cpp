@@ -4,6 +4,7 @@
 // of a given capacity.  Pure functions of the shape and the CU count; no
 // GPU is touched, so host-only checks link them directly.
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 #include "bnr_internal.h"
@@ -531,6 +532,97 @@ PrefillChoice plan_prefill_chunk(int n_tokens, int start_pos, int n_kv, int n_cu
     }
   }
   return best;
+}
+
+// Runs of a split launch.  A unit costs its key tiles plus kUnitCost (queries
+// loaded, output or state stored), and a run ends where that cost passes its
+// share; a boundary that would leave fewer than two tiles of a unit on one
+// side moves to the unit's end there.  With few units every run boundary adds
+// a state that the unit's last workgroup reads alone: for nk tiles in runs
+// of L that is L tile times and nk / L states, kStateCost tiles each, so runs
+// are no shorter than sqrt(nk kStateCost).  Of two workgroups on a CU the
+// one with issue priority (even runs) takes kEven of their share.  The
+// constants are the best of a sweep over 15 shapes (16 to 4000 tokens, 0 to
+// 4000 cached rows, 20/5 heads, MI355X): a unit cost of 2 / 3 / 4 / 6 tiles
+// takes 46 / 42 / 43 / 46 us at 1024 tokens and 281 / 267 / 259 / 259 us at
+// 4000, a shortest run of 1 / 2 / 3 tiles 33 / 29 / 30 us at 512.
+bool plan_prefill_runs(PrefillRunsArgs &a, int group, int n_cu, long long max_slots) {
+  constexpr int kUnitCost = 3;
+  constexpr double kStateCost = 0.35, kEven = 0.54, kShortest = 2.0;
+  const int uq = split_unit(group), per_cu = split_waves(group) == 4 ? 2 : 1;
+  const double even = per_cu == 2 ? 2.0 * kEven : 1.0;
+  const long long rows = (long long)a.start_pos + a.n_tokens;
+  auto nk = [&](int u) {
+    return (int)((std::min((long long)a.start_pos + (u + 1LL) * uq, rows) + 31) / 32);
+  };
+  a.n_units = (a.n_tokens + uq - 1) / uq;
+  if (a.n_units > 65535) return false;
+  const int nk_max = nk(a.n_units - 1);
+  if (nk_max > 65535) return false;
+  long long total = 0;
+  for (int u = 0; u < a.n_units; ++u) total += nk(u) + kUnitCost;
+  const double shortest = std::max(kShortest, std::sqrt(nk_max * kStateCost)) + kUnitCost;
+  long long P = std::min<long long>(std::max(1, per_cu * n_cu / a.n_kv), kMaxPrefillRuns);
+  P = std::max(1LL, std::min(P, (long long)(total / shortest)));
+  struct Cut {
+    int u, kt;
+  };
+  std::vector<Cut> cut;   // starts of the runs
+  std::vector<int> nch;   // pieces of each unit
+  for (;; P = std::max(1LL, P - std::max(1LL, P / 16))) {
+    if (per_cu == 2 && P > 1) P &= ~1LL;  // every kv head starts on a CU of its own
+    cut.assign(1, Cut{0, 0});
+    nch.assign((size_t)a.n_units, 1);
+    long long off = 0;
+    int u = 0;
+    for (long long r = 1; r < P; ++r) {
+      const long long x = (long long)(total * (double)((r / 2) * 2 + (r & 1) * even) / P);
+      while (u < a.n_units && x >= off + nk(u) + kUnitCost) off += nk(u++) + kUnitCost;
+      if (u >= a.n_units) break;
+      Cut c{u, (int)std::max(0LL, x - off - kUnitCost)};
+      if (c.kt < 2) c.kt = 0;
+      if (c.kt > nk(u) - 2 && c.kt > 0) c = Cut{u + 1, 0};
+      if (c.u >= a.n_units) break;
+      if (c.u < cut.back().u || (c.u == cut.back().u && c.kt <= cut.back().kt)) continue;
+      cut.push_back(c);
+      if (c.kt > 0) ++nch[(size_t)c.u];
+    }
+    long long slots = 0;
+    int worst = 1;
+    for (int v : nch) {
+      if (v > 1) slots += v;
+      worst = std::max(worst, v);
+    }
+    a.n_slots = (int)std::min(slots, 1LL << 20);
+    if (slots <= std::min(max_slots, 1023LL) && worst <= 255) break;
+    if (P == 1) return false;
+  }
+  a.n_runs = (int)cut.size();
+  a.grid = (a.n_kv * a.n_runs + 15) / 16 * 16;
+  std::vector<int> base((size_t)a.n_units, 0);
+  int next = 0;
+  for (int u = 0; u < a.n_units; ++u) {
+    base[(size_t)u] = next;
+    if (nch[(size_t)u] > 1) next += nch[(size_t)u];
+  }
+  std::vector<int> seen((size_t)a.n_units, 0);  // cuts inside the unit so far
+  for (int r = 0; r < a.n_runs; ++r) {
+    const Cut c = cut[(size_t)r];
+    const Cut e = r + 1 < a.n_runs ? cut[(size_t)r + 1] : Cut{a.n_units, 0};
+    long long tiles = 0;
+    int last = c.u;
+    for (int u = c.u; u < a.n_units && (u < e.u || (u == e.u && e.kt > 0)); ++u) {
+      tiles += (u == e.u ? e.kt : nk(u)) - (u == c.u ? c.kt : 0);
+      last = u;
+    }
+    if (tiles < 1 || tiles > 65535) return false;
+    const int ch = c.kt > 0 ? ++seen[(size_t)c.u] : 0;
+    a.run[r][0] = (unsigned)c.u | (unsigned)c.kt << 16;
+    a.run[r][1] = (unsigned)tiles | (unsigned)nch[(size_t)c.u] << 16 | (unsigned)ch << 24;
+    a.run[r][2] = (unsigned)base[(size_t)c.u] | (unsigned)base[(size_t)last] << 10 |
+                  (unsigned)nch[(size_t)last] << 20;
+  }
+  return true;
 }
 
 // (kv head, item) pairs a planned chunked launch may use on a cache of cap
