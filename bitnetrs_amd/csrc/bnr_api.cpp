@@ -2046,7 +2046,7 @@ int check_lm_head(size_t hidden_len, size_t weights_len, size_t scales_len, size
   return BNR_OK;
 }
 
-int run_lm_head(const float *hidden, const int8_t *w, const float *scales, float *out,
+int run_lm_head(const bnr_ctx *c, const float *hidden, const int8_t *w, const float *scales, float *out,
                 size_t vocab_size, size_t hidden_size, hipStream_t s) {
   LmHeadArgs a{};
   a.hidden = hidden;
@@ -2056,7 +2056,7 @@ int run_lm_head(const float *hidden, const int8_t *w, const float *scales, float
   a.vocab_size = (long long)vocab_size;
   a.hidden_size = (int)hidden_size;
   const bool vec = hidden_size % 16 == 0 && ((uintptr_t)w % 16) == 0 && ((uintptr_t)hidden % 16) == 0;
-  HIP_TRY(launch_lm_head_i8(a, vec, s), "lm_head launch");
+  HIP_TRY(launch_lm_head_i8(a, vec, c->n_cu, s), "lm_head launch");
   return BNR_OK;
 }
 
@@ -2089,7 +2089,7 @@ extern "C" int bnr_lm_head_matmul_i8_into(bnr_ctx *c, const float *hidden, size_
     st = put_host(c, c->d_q, {{hidden, hidden_size * 4}}, "upload hidden");
     if (st) return st;
   }
-  st = run_lm_head(c->d_q, (const int8_t *)dw, (const float *)dsc, c->d_out, vocab_size,
+  st = run_lm_head(c, c->d_q, (const int8_t *)dw, (const float *)dsc, c->d_out, vocab_size,
                    hidden_size, c->stream);
   if (st) return st;
   st = get_host(c, output, c->d_out, vocab_size * 4, "lm_head_matmul_i8_into");
@@ -2106,7 +2106,7 @@ extern "C" int bnr_dev_lm_head_matmul_i8(bnr_ctx *c, const float *hidden, const 
   if ((hidden_size && (!hidden || !weights_i8)) || !scales || !output)
     return err_backend("lm_head_matmul_i8: NULL pointer");
   DeviceGuard dg(c->device);
-  st = run_lm_head(hidden, weights_i8, scales, output, vocab_size, hidden_size, (hipStream_t)stream);
+  st = run_lm_head(c, hidden, weights_i8, scales, output, vocab_size, hidden_size, (hipStream_t)stream);
   if (st) return st;
   return set_ok();
 }

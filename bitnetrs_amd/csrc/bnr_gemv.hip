@@ -16,6 +16,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 namespace bnr {
 namespace {
 
@@ -591,10 +593,177 @@ __global__ __launch_bounds__(256) void lm_head_i8_kernel(LmHeadArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// The aligned form on the i8 matrix cores (v_mfma_i32_16x16x64_i8).  The hidden
+// vector becomes fixed point: X[k] = h[k] 2^s with |X| < 2^62, s from the
+// largest |h| (every value within 2^-38 of it keeps its 24 bits, what is cut
+// off is below 2^-61 of it), and X = sum over n < 8 of d[n] 256^n with signed
+// bytes d[n].  A product of 16 rows of weights, as they lie in memory, with the
+// digits as columns sums w d[n] exactly in int32 (2^14 K < 2^31), so the only
+// roundings are those of the eight sums to fp32 and of their scaled total:
+// 4 ulp or so, whatever K (the fp32 sums: 1.7e-7 of the result at K = 2560).
+//
+// Bound by the weights' stream.  The earlier kernel spent a conversion and an
+// FMA on every weight and read the hidden vector from LDS beside them: 57.3 us
+// = 5.7 TB/s at 128256 x 2560; here the vector unit has little to do in the
+// loop.  A wave streams whole blocks of 16 rows, 512 bytes of each per set of
+// loads, two sets in turn; the first is in flight while the workgroup forms the
+// digits.  One load instruction takes 256 consecutive bytes of four rows: in
+// the operand's own layout it would take 64 of 16 rows, half a cache line each,
+// and with the non-temporal hint the stream then ran at 4.6 TB/s (5.5 without
+// it).  The pieces change places through 4 KB of LDS per wave, chunk c of row r
+// at slot c ^ r so that neither side has bank conflicts.
+//
+// Infinities and NaN in the hidden vector (no fixed point) take plain fp32
+// sums.
+// ---------------------------------------------------------------------------
+constexpr int kLmLoads = 8;     // loads of a set: steps of 64 weights of 16 rows
+constexpr int kLmMaxK = 6144;   // digits, 8 bytes per value, beside 16 KB in 64 KB of LDS
+constexpr int kLmWgsPerCu = 4;
+typedef int int4_t __attribute__((ext_vector_type(4)));
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+void lm_head_mfma_kernel(LmHeadArgs a) {
+  extern __shared__ uint4 s_digits[];  // step ks (64 values): digit n's 64 bytes at 512 ks + 64 n
+  __shared__ uint4 s_swap[4][256];
+  __shared__ unsigned s_max[4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int n = lane & 15, u = lane >> 4;
+  const int K = a.hidden_size, chunks = (K + 64 * kLmLoads - 1) / (64 * kLmLoads);
+  const long long blocks = (a.vocab_size + 15) / 16;
+  const long long stride = (long long)gridDim.x * 4;
+  long long block = (long long)blockIdx.x * 4 + wave;
+
+  // Load i: bytes 512 c + 256 (i / 4) + 16 n of row 4 (i % 4) + u.
+  auto load = [&](int4_t (&x)[kLmLoads], long long b, int c) {
+#pragma unroll
+    for (int i = 0; i < kLmLoads; ++i) {
+      const long long row = min(16 * b + 4 * (i & 3) + u, a.vocab_size - 1);
+      // past the row: its last bytes (their digits are zero)
+      const int k = min(512 * c + 256 * (i >> 2) + 16 * n, K - 16);
+      x[i] = __builtin_nontemporal_load(reinterpret_cast<const int4_t *>(a.weight + row * K + k));
+    }
+  };
+  int4_t wa[kLmLoads], wb[kLmLoads];
+  load(wa, min(block, blocks - 1), 0);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // Digits of the hidden vector, four values per thread and round.
+  const int quads = chunks * kLmLoads * 16;
+  unsigned mx = 0;
+  for (int q = tid; 4 * q < K; q += 256) {
+    const uint4 h = *reinterpret_cast<const uint4 *>(a.hidden + 4 * q);
+    mx = max(mx, max(max(h.x & 0x7fffffffu, h.y & 0x7fffffffu), max(h.z & 0x7fffffffu, h.w & 0x7fffffffu)));
+  }
+  for (int m = 1; m < 64; m <<= 1) mx = max(mx, (unsigned)__shfl_xor((int)mx, m));
+  if (lane == 0) s_max[wave] = mx;
+  __syncthreads();
+  mx = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
+  if (mx >= 0x7f800000u) {  // uniform over the grid
+    for (; block < blocks; block += stride)
+      for (int r = 0; r < 16; ++r) {
+        const long long row = 16 * block + r;
+        if (row >= a.vocab_size) break;
+        float acc = 0.f;
+        for (int k = lane; k < K; k += 64) acc = fmaf((float)a.weight[row * K + k], a.hidden[k], acc);
+        for (int m = 1; m < 64; m <<= 1) acc += __shfl_xor(acc, m);
+        if (lane == 0) a.out[row] = acc * a.scales[row];
+      }
+    return;
+  }
+  const int e_max = max((int)(mx >> 23), 1);
+  unsigned *digits = reinterpret_cast<unsigned *>(s_digits);
+  for (int q = tid; q < quads; q += 256) {
+    const uint4 h = 4 * q < K ? *reinterpret_cast<const uint4 *>(a.hidden + 4 * q) : make_uint4(0, 0, 0, 0);
+    const unsigned hb[4] = {h.x, h.y, h.z, h.w};
+    unsigned lo[4], hi[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int ef = (int)(hb[i] >> 23 & 255u);
+      const long long m = (long long)((hb[i] & 0x7fffffu) | (ef ? 0x800000u : 0u));
+      const int sh = 38 - (e_max - max(ef, 1));
+      long long x = sh >= 0 ? m << sh : m >> min(-sh, 63);
+      x = (hb[i] >> 31) ? -x : x;
+      // signed bytes: add 128 to the lower seven with their carries, then take it off each
+      const unsigned long long C = 0x0080808080808080ull;
+      const unsigned long long d = ((unsigned long long)x + C) ^ C;
+      lo[i] = (unsigned)d;
+      hi[i] = (unsigned)(d >> 32);
+    }
+    const uint4 d0 = transpose_bytes(make_uint4(lo[0], lo[1], lo[2], lo[3]));
+    const uint4 d4 = transpose_bytes(make_uint4(hi[0], hi[1], hi[2], hi[3]));
+    unsigned *p = digits + (q >> 4) * 128 + (q & 15);
+    p[0] = d0.x;
+    p[16] = d0.y;
+    p[32] = d0.z;
+    p[48] = d0.w;
+    p[64] = d4.x;
+    p[80] = d4.y;
+    p[96] = d4.z;
+    p[112] = d4.w;
+  }
+  __syncthreads();
+
+  // Column n and n + 8 both hold digit n % 8.
+  const uint4 *op = s_digits + (n & 7) * 4 + u;
+  const int ex = 8 * (n & 7) + e_max - 188;
+  int4_t *swap = reinterpret_cast<int4_t *>(s_swap[wave]);
+  int4_t *put = swap + 16 * u;  // row 4 j + u at 64 j + 16 u
+  const int4_t *get = swap + 16 * n;
+  int4_t acc = {0, 0, 0, 0};
+  int c = 0;
+  auto chunk = [&](int4_t (&cur)[kLmLoads], int4_t (&nxt)[kLmLoads]) {
+    const int cn = c + 1 < chunks ? c + 1 : 0;
+    const long long bn = cn ? block : block + stride;
+    if (bn < blocks) load(nxt, bn, cn);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < kLmLoads; i += 4) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) put[64 * j + (n ^ (4 * j + u))] = cur[i + j];
+      __builtin_amdgcn_wave_barrier();  // the wave's own LDS operations keep their order
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int4_t w = get[(4 * j + u) ^ n];
+        const int4_t d = __builtin_bit_cast(int4_t, op[(kLmLoads * c + i + j) * 32]);
+        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(w, d, acc, 0, 0, 0);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+    if (cn == 0) {
+      // rows 16 block + 4 u + r: the eight digits' sums, scaled, added over the lanes
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float v = ldexpf((float)acc[r], ex);
+        v += dppf<0xB1>(v);
+        v += dppf<0x4E>(v);
+        v += dppf<0x141>(v);
+        const long long row = 16 * block + 4 * u + r;
+        if (n == r && row < a.vocab_size) a.out[row] = v * a.scales[row];
+      }
+      acc = int4_t{0, 0, 0, 0};
+    }
+    c = cn;
+    block = bn;
+  };
+  while (block < blocks) {
+    chunk(wa, wb);
+    if (block >= blocks) break;
+    chunk(wb, wa);
+  }
+}
+
 }  // namespace
 
-hipError_t launch_lm_head_i8(const LmHeadArgs &a, bool vec, hipStream_t s) {
+hipError_t launch_lm_head_i8(const LmHeadArgs &a, bool vec, int n_cu, hipStream_t s) {
   if (a.vocab_size <= 0) return hipSuccess;
+  if (vec && a.hidden_size >= 16 && a.hidden_size <= kLmMaxK) {
+    const long long blocks = (a.vocab_size + 15) / 16;
+    const int chunks = (a.hidden_size + 64 * kLmLoads - 1) / (64 * kLmLoads);
+    const long long wgs = std::min<long long>((blocks + 3) / 4, (long long)kLmWgsPerCu * n_cu);
+    lm_head_mfma_kernel<<<dim3((unsigned)wgs), dim3(256), (size_t)chunks * kLmLoads * 512, s>>>(a);
+    return hipGetLastError();
+  }
   const long long rows_per_wg = 16 * kLmBlocks;
   const dim3 grid((unsigned)((a.vocab_size + rows_per_wg - 1) / rows_per_wg));
   if (vec)

@@ -648,7 +648,7 @@ struct LmHeadArgs {
   int hidden_size;
 };
 // vec: 16-byte aligned weights with hidden_size % 16 == 0, hidden 16-byte aligned.
-hipError_t launch_lm_head_i8(const LmHeadArgs &a, bool vec, hipStream_t s);
+hipError_t launch_lm_head_i8(const LmHeadArgs &a, bool vec, int n_cu, hipStream_t s);
 
 // Layer glue (bnr_glue.hip).
 struct NormQuantArgs {

@@ -82,3 +82,59 @@ def test_lm_head_shape_errors_match_oracle(backend):
         with pytest.raises(bitnetrs_amd.InvalidShape) as ge:
             backend.lm_head_matmul_i8_into(*a)
         assert str(ge.value) == str(oe.value)
+
+
+@pytest.mark.parametrize("v,h,kind", [(1, 16, "normal"), (17, 48, "normal"), (63, 512, "normal"),
+                                      (4100, 528, "wide"), (70000, 1040, "outlier"), (33, 6144, "wide"),
+                                      (20, 6160, "normal"), (65, 2560, "tiny"), (65, 2560, "zero")])
+def test_device_lm_head_digits(backend, v, h, kind):
+    """The i8 matrix-core form at its edges -- one row, part of a block, several
+    blocks per wave, K within and past a set of loads, its largest K and the
+    form beyond it -- and over magnitudes: values 2^-40 to 1, one value 2^30
+    times the others (and zero weights there, so that the rest must survive),
+    subnormals, zeros.  fp32 sums would be off by up to K ulp of the products'
+    magnitude; eight exact sums rounded once are off by a few."""
+    case(f"lm head digits vocab {v} hidden {h} {kind}")
+    import torch
+
+    hid, w, sc = workload(v + h, v, h)
+    rng = np.random.default_rng(h)
+    if kind == "wide":
+        hid = (hid * np.exp2(rng.integers(-40, 1, size=h))).astype(f32)
+    elif kind == "outlier":
+        hid[5] = 2.0 ** 30
+        w[:, 5] = 0
+    elif kind == "tiny":
+        hid = (hid * 1e-40).astype(f32)
+    elif kind == "zero":
+        hid[:] = 0
+    out = torch.full((v,), float("nan"), device="cuda")
+    backend.dev_lm_head_matmul_i8(torch.from_numpy(hid).cuda(), torch.from_numpy(w.reshape(-1)).cuda(),
+                                  torch.from_numpy(sc).cuda(), out, v, h)
+    torch.cuda.synchronize()
+    exact = (w.astype(np.float64) @ hid.astype(np.float64)) * sc
+    mag = (np.abs(w).astype(np.float64) @ np.abs(hid).astype(np.float64)) * sc
+    # 8 roundings of digit sums (the largest at most twice the products'
+    # magnitude), 3 additions, the scale; beyond 6144 values the fp32 sums
+    ulps = 16 if h <= 6144 else 4 * h
+    cut = h * 128 * np.abs(hid).max() * 2.0 ** -61 * sc  # below the last digit
+    assert np.all(np.abs(out.cpu().numpy() - exact) <= ulps * 2.0 ** -24 * mag + cut + 1e-44)
+
+
+def test_device_lm_head_non_finite(backend):
+    """An infinity or a NaN in the hidden vector: what fp32 sums give."""
+    case("lm head non-finite hidden")
+    import torch
+
+    v, h = 100, 256
+    hid, w, sc = workload(3, v, h)
+    w[:, 9] = np.arange(v) % 3 - 1  # -, 0, + at the infinity
+    for bad in (np.inf, -np.inf, np.nan):
+        hid[9] = bad
+        out = torch.zeros(v, device="cuda")
+        backend.dev_lm_head_matmul_i8(torch.from_numpy(hid).cuda(), torch.from_numpy(w.reshape(-1)).cuda(),
+                                      torch.from_numpy(sc).cuda(), out, v, h)
+        torch.cuda.synchronize()
+        with np.errstate(invalid="ignore"):
+            want = w[:, 9].astype(np.float64) * bad
+        np.testing.assert_array_equal(out.cpu().numpy(), want.astype(f32))
