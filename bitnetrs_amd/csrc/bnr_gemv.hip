@@ -38,20 +38,23 @@ constexpr int kGroups = kPass / 16;         // 16-activation groups per pass
 constexpr int kPieces = kPass / 64;         // 16-byte weight pieces per row and pass
 constexpr int kPiecesPerLane = kPieces / 16;
 
-// Decode table for v_perm_b32: byte c of kCodeValue is the int8 value of
-// code c (+1, 0, -1, 0).
-constexpr unsigned kCodeValue = 0x00FF0001u;
+// Decode tables for v_perm_b32, whose selector bytes 0 .. 3 take that byte of
+// the table, 4 .. 7 a byte of a zero word, 8 the sign of the table's byte 1 and
+// 12 zero.  For codes in bits 0 and 1 of a byte (selectors 0 .. 3) byte c of
+// kCodeLow is the int8 value of code c (+1, 0, -1, 0); for codes left in bits 2
+// and 3 (selectors 0, 4, 8, 12) kCodeHigh gives the same values.
+constexpr unsigned kCodeLow = 0x00FF0001u, kCodeHigh = 0x00008001u;
 
 // One packed dword w = weights 16g .. 16g+15 (weight 16g + 4k + p at bits
-// 8k + 2p).  (w >> 2p) & 0x03030303 puts the codes of weights 4k + p,
-// k = 0..3, in its four bytes; v_perm maps each code to its value.  act.{x,y,z,w}
-// hold the activations of the same positions for p = 0, 1, 2, 3.
+// 8k + 2p): the codes of weights 4k + p, k = 0..3, are masked out of its four
+// bytes (p = 0 and 1 of w, 2 and 3 of w >> 4) and mapped to their values.
+// act.{x,y,z,w} hold the activations of the same positions for p = 0, 1, 2, 3.
 __device__ __forceinline__ int dot16(unsigned w, uint4 act, int acc) {
-  const unsigned m = 0x03030303u;
-  acc = __builtin_amdgcn_sdot4((int)__builtin_amdgcn_perm(0u, kCodeValue, w & m), (int)act.x, acc, false);
-  acc = __builtin_amdgcn_sdot4((int)__builtin_amdgcn_perm(0u, kCodeValue, (w >> 2) & m), (int)act.y, acc, false);
-  acc = __builtin_amdgcn_sdot4((int)__builtin_amdgcn_perm(0u, kCodeValue, (w >> 4) & m), (int)act.z, acc, false);
-  acc = __builtin_amdgcn_sdot4((int)__builtin_amdgcn_perm(0u, kCodeValue, (w >> 6) & m), (int)act.w, acc, false);
+  const unsigned lo = 0x03030303u, hi = 0x0C0C0C0Cu, v = w >> 4;
+  acc = __builtin_amdgcn_sdot4((int)__builtin_amdgcn_perm(0u, kCodeLow, w & lo), (int)act.x, acc, false);
+  acc = __builtin_amdgcn_sdot4((int)__builtin_amdgcn_perm(0u, kCodeHigh, w & hi), (int)act.y, acc, false);
+  acc = __builtin_amdgcn_sdot4((int)__builtin_amdgcn_perm(0u, kCodeLow, v & lo), (int)act.z, acc, false);
+  acc = __builtin_amdgcn_sdot4((int)__builtin_amdgcn_perm(0u, kCodeHigh, v & hi), (int)act.w, acc, false);
   return acc;
 }
 
@@ -263,7 +266,7 @@ __device__ __forceinline__ float norm_y(float x, float inv, float g) {
   return x * inv * g;
 }
 
-template <bool VEC, int NG, int LPR>
+template <int NG, int LPR>
 __global__ __launch_bounds__(256) void ternary_gemv_norm_kernel(TernaryGemvGroupArgs a,
                                                                 GemvNormArgs p) {
   constexpr int kNormGroupsPerThread = NG;
@@ -291,68 +294,22 @@ __global__ __launch_bounds__(256) void ternary_gemv_norm_kernel(TernaryGemvGroup
   const int K = a.in_features, nb = (K + 3) / 4;
   const int row = (b - off) * kRows + slot;
   const long long b0 = (long long)min(row, m - 1) * a.packed_cols;
-  // 1. x for groups tid, tid+256 (16 consecutive elements each) and gamma,
-  // loaded before the weights: loads return in order, so these small,
-  // cache-resident vectors arrive first and the prologue runs while the
-  // weights are still in flight.  VEC: K % 16 == 0 and 16-byte aligned
-  // vectors, so a group is four float4 loads of each input.
   float x[kNormGroupsPerThread][16], g[kNormGroupsPerThread][16];
-  float4 xa[VEC ? kNormGroupsPerThread : 1][4], xb[VEC ? kNormGroupsPerThread : 1][4],
-      xg[VEC ? kNormGroupsPerThread : 1][4];
-  if (VEC) {
-    // One batch of loads, no branches between them: the second operand is a
-    // itself when the mode has none; groups past K read group 0 (discarded).
-    const float *pb = p.mode == kGluePlain ? p.a : p.b;
-#pragma unroll
-    for (int q = 0; q < kNormGroupsPerThread; ++q) {
-      const int e0 = 16 * (tid + 256 * q);
-      const int base = e0 < K ? e0 : 0;
-#pragma unroll
-      for (int v4 = 0; v4 < 4; ++v4) {
-        xa[q][v4] = *reinterpret_cast<const float4 *>(p.a + base + 4 * v4);
-        xb[q][v4] = *reinterpret_cast<const float4 *>(pb + base + 4 * v4);
-        xg[q][v4] = *reinterpret_cast<const float4 *>(p.gamma + base + 4 * v4);
-      }
-    }
-  }
-  __builtin_amdgcn_sched_barrier(0);  // keep the activation loads ahead of the weights
   // 2. this lane's weight pieces (in flight during the prologue)
   uint4 wq[kNormPiecesPerLane];
 #pragma unroll
   for (int i = 0; i < kNormPiecesPerLane; ++i) {
     const int c = j + LPR * i;
-    if (VEC)
-      wq[i] = 16 * c < nb ? ld16_nt(w + b0 + 16 * c) : make_uint4(0, 0, 0, 0);
-    else
-      wq[i] = 16 * c < nb ? load16_bounded(w, b0 + 16 * c, b0 + nb) : make_uint4(0, 0, 0, 0);
+    wq[i] = 16 * c < nb ? load16_bounded(w, b0 + 16 * c, b0 + nb) : make_uint4(0, 0, 0, 0);
   }
-  if (VEC) {
 #pragma unroll
-    for (int q = 0; q < kNormGroupsPerThread; ++q) {
-      const bool in = 16 * (tid + 256 * q) < K;
+  for (int q = 0; q < kNormGroupsPerThread; ++q) {
+    const int e0 = 16 * (tid + 256 * q);
 #pragma unroll
-      for (int v4 = 0; v4 < 4; ++v4) {
-        const float4 u = xa[q][v4], v = xb[q][v4], gv = xg[q][v4];
-        x[q][4 * v4] = in ? norm_x_of(p.mode, u.x, v.x) : 0.f;
-        x[q][4 * v4 + 1] = in ? norm_x_of(p.mode, u.y, v.y) : 0.f;
-        x[q][4 * v4 + 2] = in ? norm_x_of(p.mode, u.z, v.z) : 0.f;
-        x[q][4 * v4 + 3] = in ? norm_x_of(p.mode, u.w, v.w) : 0.f;
-        g[q][4 * v4] = in ? gv.x : 0.f;
-        g[q][4 * v4 + 1] = in ? gv.y : 0.f;
-        g[q][4 * v4 + 2] = in ? gv.z : 0.f;
-        g[q][4 * v4 + 3] = in ? gv.w : 0.f;
-      }
-    }
-  } else {
-#pragma unroll
-    for (int q = 0; q < kNormGroupsPerThread; ++q) {
-      const int e0 = 16 * (tid + 256 * q);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int i = e0 + e;
-        x[q][e] = i < K ? norm_x(p, i) : 0.f;
-        g[q][e] = i < K ? p.gamma[i] : 0.f;
-      }
+    for (int e = 0; e < 16; ++e) {
+      const int i = e0 + e;
+      x[q][e] = i < K ? norm_x(p, i) : 0.f;
+      g[q][e] = i < K ? p.gamma[i] : 0.f;
     }
   }
   // 3. sum of squares
@@ -365,17 +322,9 @@ __global__ __launch_bounds__(256) void ternary_gemv_norm_kernel(TernaryGemvGroup
 #pragma unroll
     for (int q = 0; q < kNormGroupsPerThread; ++q) {
       const int e0 = 16 * (tid + 256 * q);
-      if (VEC) {
-        if (e0 < K)
 #pragma unroll
-          for (int v4 = 0; v4 < 4; ++v4)
-            *reinterpret_cast<float4 *>(p.h_out + e0 + 4 * v4) =
-                make_float4(x[q][4 * v4], x[q][4 * v4 + 1], x[q][4 * v4 + 2], x[q][4 * v4 + 3]);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 16; ++e)
-          if (e0 + e < K) p.h_out[e0 + e] = x[q][e];
-      }
+      for (int e = 0; e < 16; ++e)
+        if (e0 + e < K) p.h_out[e0 + e] = x[q][e];
     }
   }
   // block sum (4 waves); the same tree in every workgroup
@@ -434,6 +383,156 @@ __global__ __launch_bounds__(256) void ternary_gemv_norm_kernel(TernaryGemvGroup
   if (j == 0 && row < m) out[row] = (float)acc * cs;
 }
 
+// int8 of v: round half away from zero, clamped.  trunc(v + 0.5 - 2^-25 with
+// v's sign) is roundf(v) for |v| < 2^22: the sum of a half-way value rounds up
+// to the next integer, that of the float below it does not.
+__device__ __forceinline__ unsigned quant_byte(float v) {
+  const float r = v + copysignf(0x1.fffffep-2f, v);
+  return (unsigned)((int)fminf(fmaxf(r, -128.0f), 127.0f)) & 0xFFu;
+}
+
+// The aligned form (K % 64 == 0, 16-byte aligned rows and vectors).  Thread t
+// forms the quads t, t + 256, ... of the activations (NQ >= K / 1024 of them):
+// a wave's load takes 1 KB in a row.  The four lanes that hold a group of 16
+// exchange bytes (two quad permutes) so that each stores one of the group's
+// four dwords for dot16.  Everything before the weights are there is latency:
+// three vectors from the other side of a kernel boundary, two block
+// reductions; everything after is the decode.  Per launch of the two in a 2B
+// feed-forward layer: 7.46 us with 16 consecutive activations per thread (a
+// load then took 16 bytes of 64 lines, and half the threads had none at K =
+// 2560) and the library's roundf, %NEW% us here.
+template <int NQ, int LPR>
+__global__ __launch_bounds__(256) void ternary_gemv_norm_vec_kernel(TernaryGemvGroupArgs a,
+                                                                    GemvNormArgs p) {
+  constexpr int kPcs = 16 * NQ;                    // 16-byte weight pieces per row
+  constexpr int kPcsPerLane = (kPcs + LPR - 1) / LPR;
+  constexpr int kRows = 256 / LPR;
+  __shared__ unsigned s_act[16 * kPcs];  // group g: 4 dwords at 4 ((g % 4) kPcs + g / 4)
+  __shared__ float red[8];
+  const int tid = threadIdx.x, slot = tid / LPR, j = tid % LPR, lane = tid & 63, wave = tid >> 6;
+  const int b = blockIdx.x;
+  const uint8_t *w = a.weight[0];
+  float *out = a.out[0];
+  float ws = a.weight_scale[0];
+  int m = a.out_features[0], off = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxGemvGroup; ++i) {
+    if (i < a.n && b >= a.wg_off[i]) {
+      w = a.weight[i];
+      out = a.out[i];
+      ws = a.weight_scale[i];
+      m = a.out_features[i];
+      off = a.wg_off[i];
+    }
+  }
+  const int K = a.in_features, quads = K / 4, pcs = K / 64;
+  const int row = (b - off) * kRows + slot;
+  // 1. the activations' loads, ahead of the weights: loads return in order.
+  // No branches between them: the second operand is a itself when the mode
+  // has none; quads past K read quad 0 (discarded).
+  const float *pb = p.mode == kGluePlain ? p.a : p.b;
+  float4 xa[NQ], xb[NQ], xg[NQ];
+#pragma unroll
+  for (int i = 0; i < NQ; ++i) {
+    const int q = tid + 256 * i, o = q < quads ? 4 * q : 0;
+    xa[i] = *reinterpret_cast<const float4 *>(p.a + o);
+    xb[i] = *reinterpret_cast<const float4 *>(pb + o);
+    xg[i] = *reinterpret_cast<const float4 *>(p.gamma + o);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  // 2. this lane's weight pieces (in flight during the prologue)
+  const uint8_t *wrow = w + (long long)min(row, m - 1) * a.packed_cols;
+  uint4 wq[kPcsPerLane];
+#pragma unroll
+  for (int i = 0; i < kPcsPerLane; ++i) {
+    const int c = j + LPR * i;
+    wq[i] = c < pcs ? ld16_nt(wrow + 16 * c) : make_uint4(0, 0, 0, 0);
+  }
+  // 3. x, its sum of squares; the same tree in every workgroup
+  float x[NQ][4], ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NQ; ++i) {
+    const bool in = tid + 256 * i < quads;
+    x[i][0] = in ? norm_x_of(p.mode, xa[i].x, xb[i].x) : 0.f;
+    x[i][1] = in ? norm_x_of(p.mode, xa[i].y, xb[i].y) : 0.f;
+    x[i][2] = in ? norm_x_of(p.mode, xa[i].z, xb[i].z) : 0.f;
+    x[i][3] = in ? norm_x_of(p.mode, xa[i].w, xb[i].w) : 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss = fmaf(x[i][e], x[i][e], ss);
+  }
+  if (p.h_out && b == 0) {
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      const int q = tid + 256 * i;
+      if (q < quads)
+        *reinterpret_cast<float4 *>(p.h_out + 4 * q) = make_float4(x[i][0], x[i][1], x[i][2], x[i][3]);
+    }
+  }
+  ss = wave_sum_f(ss);
+  if (lane == 0) red[wave] = ss;
+  __syncthreads();
+  const float sum_sq = (red[0] + red[1]) + (red[2] + red[3]);
+  const float inv = 1.0f / sqrtf(sum_sq / (float)K + p.eps);
+  float mx = 0.f;
+#pragma unroll
+  for (int i = 0; i < NQ; ++i) {
+    const float g[4] = {xg[i].x, xg[i].y, xg[i].z, xg[i].w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      x[i][e] = tid + 256 * i < quads ? norm_y(x[i][e], inv, g[e]) : 0.f;
+      mx = fmaxf(mx, fabsf(x[i][e]));
+    }
+  }
+  mx = wave_max_f(mx);
+  if (lane == 0) red[4 + wave] = mx;
+  __syncthreads();
+  const float mm = fmaxf(fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7])), 1e-5f);
+  const float scale = mm / 127.0f, inv_scale = 127.0f / mm;
+  // 4. int8 activations: lane 4g + t holds activations 4t .. 4t+3 of its
+  // group, and stores dword t: activations t, 4+t, 8+t, 12+t.
+  const unsigned sel1 = (lane & 1) ? 0x03070105u : 0x06020400u;
+  const unsigned sel2 = (lane & 2) ? 0x03020706u : 0x05040100u;
+#pragma unroll
+  for (int i = 0; i < NQ; ++i) {
+    unsigned d = quant_byte(x[i][0] * inv_scale) | quant_byte(x[i][1] * inv_scale) << 8 |
+                 quant_byte(x[i][2] * inv_scale) << 16 | quant_byte(x[i][3] * inv_scale) << 24;
+    d = __builtin_amdgcn_perm((unsigned)dpp_i<0xB1>((int)d), d, sel1);  // lane ^ 1
+    d = __builtin_amdgcn_perm((unsigned)dpp_i<0x4E>((int)d), d, sel2);  // lane ^ 2
+    const int q = tid + 256 * i, g = q >> 2;
+    s_act[4 * ((g & 3) * kPcs + (g >> 2)) + (q & 3)] = d;
+  }
+  __syncthreads();
+  // 5. the projection
+  const uint4 *act = reinterpret_cast<const uint4 *>(s_act);
+  int acc = 0;
+#pragma unroll
+  for (int i = 0; i < kPcsPerLane; ++i) {
+    const int c = j + LPR * i;
+    if (c < pcs) {
+      acc = dot16(wq[i].x, act[c], acc);
+      acc = dot16(wq[i].y, act[kPcs + c], acc);
+      acc = dot16(wq[i].z, act[2 * kPcs + c], acc);
+      acc = dot16(wq[i].w, act[3 * kPcs + c], acc);
+    }
+  }
+  acc = lane_group_sum_i<LPR>(acc);
+  // combined_scale = weight_scale * act_scale / 127.0 (gemv.rs:297), act_scale = scale * 127
+  const float t = ws * (scale * 127.0f);
+  const float cs = t / 127.0f;
+  if (j == 0 && row < m) out[row] = (float)acc * cs;
+}
+
+template <int LPR>
+hipError_t launch_norm_vec(const TernaryGemvGroupArgs &a, const GemvNormArgs &p, int wgs, hipStream_t s) {
+  const dim3 grid(wgs), block(256);
+  const int nq = (a.in_features + 1023) / 1024;
+  if (nq <= 3) ternary_gemv_norm_vec_kernel<3, LPR><<<grid, block, 0, s>>>(a, p);
+  else if (nq <= 4) ternary_gemv_norm_vec_kernel<4, LPR><<<grid, block, 0, s>>>(a, p);
+  else if (nq <= 7) ternary_gemv_norm_vec_kernel<7, LPR><<<grid, block, 0, s>>>(a, p);
+  else ternary_gemv_norm_vec_kernel<8, LPR><<<grid, block, 0, s>>>(a, p);
+  return hipGetLastError();
+}
+
 }  // namespace
 
 hipError_t launch_ternary_gemv_norm(const TernaryGemvGroupArgs &a, const GemvNormArgs &p, bool vec,
@@ -441,21 +540,20 @@ hipError_t launch_ternary_gemv_norm(const TernaryGemvGroupArgs &a, const GemvNor
   const int wgs = a.wg_off[a.n];
   if (wgs <= 0) return hipSuccess;
   if (a.in_features > kNormK) return hipErrorInvalidValue;
+  if (vec) {
+    switch (p.rows) {
+      case 16: return launch_norm_vec<16>(a, p, wgs, s);
+      case 32: return launch_norm_vec<8>(a, p, wgs, s);
+      case 64: return launch_norm_vec<4>(a, p, wgs, s);
+      default: return hipErrorInvalidValue;
+    }
+  }
   const bool one = a.in_features <= kNormK / 2;
   auto go = [&](auto kern) { kern<<<dim3(wgs), dim3(256), 0, s>>>(a, p); };
   switch (p.rows) {
-    case 16:
-      if (vec) one ? go(ternary_gemv_norm_kernel<true, 1, 16>) : go(ternary_gemv_norm_kernel<true, 2, 16>);
-      else one ? go(ternary_gemv_norm_kernel<false, 1, 16>) : go(ternary_gemv_norm_kernel<false, 2, 16>);
-      break;
-    case 32:
-      if (vec) one ? go(ternary_gemv_norm_kernel<true, 1, 8>) : go(ternary_gemv_norm_kernel<true, 2, 8>);
-      else one ? go(ternary_gemv_norm_kernel<false, 1, 8>) : go(ternary_gemv_norm_kernel<false, 2, 8>);
-      break;
-    case 64:
-      if (vec) one ? go(ternary_gemv_norm_kernel<true, 1, 4>) : go(ternary_gemv_norm_kernel<true, 2, 4>);
-      else one ? go(ternary_gemv_norm_kernel<false, 1, 4>) : go(ternary_gemv_norm_kernel<false, 2, 4>);
-      break;
+    case 16: one ? go(ternary_gemv_norm_kernel<1, 16>) : go(ternary_gemv_norm_kernel<2, 16>); break;
+    case 32: one ? go(ternary_gemv_norm_kernel<1, 8>) : go(ternary_gemv_norm_kernel<2, 8>); break;
+    case 64: one ? go(ternary_gemv_norm_kernel<1, 4>) : go(ternary_gemv_norm_kernel<2, 4>); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
