@@ -302,7 +302,7 @@ struct bnr_ctx {
   int pf_balanced = -1;           // balanced key chunks: -1 planner, 0 never, 1 always
   // norm-fused GEMV: the most rows per workgroup (16, 32, 64) that keep the
   // launch at or above this many workgroups
-  int gemv_norm_min_wgs = 256;
+  int gemv_norm_min_wgs = 128;
   int pf_pair = -1;               // paired 16-query launches: -1 planner (4 q heads per kv head), 0 never, 1 where possible
   int pf_split = -1;              // fp16-pair prefill: -1 by shape unless another launch is forced, 0 never, 1 wherever it fits
   std::vector<PrefillPlanEntry> pf_plans;  // recent (shape -> key tiles per chunk) plans

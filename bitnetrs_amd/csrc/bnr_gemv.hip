@@ -99,6 +99,14 @@ __device__ __forceinline__ int lane_group_sum_i(int v) {
   v += dpp_i<0x4E>(v);
   if (L >= 8) v += dpp_i<0x141>(v);
   if (L >= 16) v += dpp_i<0x140>(v);
+  if (L >= 32) {
+    const auto r = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+    v = (int)((unsigned)r[0] + (unsigned)r[1]);
+  }
+  if (L >= 64) {
+    const auto r = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+    v = (int)((unsigned)r[0] + (unsigned)r[1]);
+  }
   return v;
 }
 
@@ -399,16 +407,23 @@ __device__ __forceinline__ unsigned quant_byte(float v) {
 // three vectors from the other side of a kernel boundary, two block
 // reductions; everything after is the decode.  Per launch of the two in a 2B
 // feed-forward layer: 7.46 us with 16 consecutive activations per thread (a
-// load then took 16 bytes of 64 lines, and half the threads had none at K =
-// 2560) and the library's roundf, %NEW% us here.
-template <int NQ, int LPR>
-__global__ __launch_bounds__(256) void ternary_gemv_norm_vec_kernel(TernaryGemvGroupArgs a,
+// load then took 16 bytes of 64 lines, and 96 of the threads had none at K =
+// 2560) and the library's roundf, 6.33 us with quads and 256 threads, 6.1 us
+// with the workgroups below.
+//
+// T threads, LPR lanes per row: 16 or 32 rows in 256 threads; 64 rows in 512,
+// where the launch is that long (gate + up: 216 workgroups read the vectors
+// instead of 432, 6.4 -> 6.2 us on the average of gate + up and down); 16 rows
+// in 512 past K = 4096, where the vectors are most of the prologue (down: 30
+// layers 3 us less; q/k/v and o, at K = 2560, lose 0.4 us each in 512).
+template <int NQ, int LPR, int T>
+__global__ __launch_bounds__(T) void ternary_gemv_norm_vec_kernel(TernaryGemvGroupArgs a,
                                                                     GemvNormArgs p) {
-  constexpr int kPcs = 16 * NQ;                    // 16-byte weight pieces per row
+  constexpr int kPcs = NQ * T / 16;  // 16-byte weight pieces per row
   constexpr int kPcsPerLane = (kPcs + LPR - 1) / LPR;
-  constexpr int kRows = 256 / LPR;
+  constexpr int kRows = T / LPR, kWaves = T / 64;
   __shared__ unsigned s_act[16 * kPcs];  // group g: 4 dwords at 4 ((g % 4) kPcs + g / 4)
-  __shared__ float red[8];
+  __shared__ float red[2][kWaves];
   const int tid = threadIdx.x, slot = tid / LPR, j = tid % LPR, lane = tid & 63, wave = tid >> 6;
   const int b = blockIdx.x;
   const uint8_t *w = a.weight[0];
@@ -434,7 +449,7 @@ __global__ __launch_bounds__(256) void ternary_gemv_norm_vec_kernel(TernaryGemvG
   float4 xa[NQ], xb[NQ], xg[NQ];
 #pragma unroll
   for (int i = 0; i < NQ; ++i) {
-    const int q = tid + 256 * i, o = q < quads ? 4 * q : 0;
+    const int q = tid + T * i, o = q < quads ? 4 * q : 0;
     xa[i] = *reinterpret_cast<const float4 *>(p.a + o);
     xb[i] = *reinterpret_cast<const float4 *>(pb + o);
     xg[i] = *reinterpret_cast<const float4 *>(p.gamma + o);
@@ -452,7 +467,7 @@ __global__ __launch_bounds__(256) void ternary_gemv_norm_vec_kernel(TernaryGemvG
   float x[NQ][4], ss = 0.f;
 #pragma unroll
   for (int i = 0; i < NQ; ++i) {
-    const bool in = tid + 256 * i < quads;
+    const bool in = tid + T * i < quads;
     x[i][0] = in ? norm_x_of(p.mode, xa[i].x, xb[i].x) : 0.f;
     x[i][1] = in ? norm_x_of(p.mode, xa[i].y, xb[i].y) : 0.f;
     x[i][2] = in ? norm_x_of(p.mode, xa[i].z, xb[i].z) : 0.f;
@@ -463,15 +478,17 @@ __global__ __launch_bounds__(256) void ternary_gemv_norm_vec_kernel(TernaryGemvG
   if (p.h_out && b == 0) {
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
-      const int q = tid + 256 * i;
+      const int q = tid + T * i;
       if (q < quads)
         *reinterpret_cast<float4 *>(p.h_out + 4 * q) = make_float4(x[i][0], x[i][1], x[i][2], x[i][3]);
     }
   }
   ss = wave_sum_f(ss);
-  if (lane == 0) red[wave] = ss;
+  if (lane == 0) red[0][wave] = ss;
   __syncthreads();
-  const float sum_sq = (red[0] + red[1]) + (red[2] + red[3]);
+  float sum_sq = 0.f;
+#pragma unroll
+  for (int i = 0; i < kWaves; ++i) sum_sq += red[0][i];
   const float inv = 1.0f / sqrtf(sum_sq / (float)K + p.eps);
   float mx = 0.f;
 #pragma unroll
@@ -479,14 +496,16 @@ __global__ __launch_bounds__(256) void ternary_gemv_norm_vec_kernel(TernaryGemvG
     const float g[4] = {xg[i].x, xg[i].y, xg[i].z, xg[i].w};
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      x[i][e] = tid + 256 * i < quads ? norm_y(x[i][e], inv, g[e]) : 0.f;
+      x[i][e] = tid + T * i < quads ? norm_y(x[i][e], inv, g[e]) : 0.f;
       mx = fmaxf(mx, fabsf(x[i][e]));
     }
   }
   mx = wave_max_f(mx);
-  if (lane == 0) red[4 + wave] = mx;
+  if (lane == 0) red[1][wave] = mx;
   __syncthreads();
-  const float mm = fmaxf(fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7])), 1e-5f);
+  float mm = 1e-5f;
+#pragma unroll
+  for (int i = 0; i < kWaves; ++i) mm = fmaxf(mm, red[1][i]);
   const float scale = mm / 127.0f, inv_scale = 127.0f / mm;
   // 4. int8 activations: lane 4g + t holds activations 4t .. 4t+3 of its
   // group, and stores dword t: activations t, 4+t, 8+t, 12+t.
@@ -498,7 +517,7 @@ __global__ __launch_bounds__(256) void ternary_gemv_norm_vec_kernel(TernaryGemvG
                  quant_byte(x[i][2] * inv_scale) << 16 | quant_byte(x[i][3] * inv_scale) << 24;
     d = __builtin_amdgcn_perm((unsigned)dpp_i<0xB1>((int)d), d, sel1);  // lane ^ 1
     d = __builtin_amdgcn_perm((unsigned)dpp_i<0x4E>((int)d), d, sel2);  // lane ^ 2
-    const int q = tid + 256 * i, g = q >> 2;
+    const int q = tid + T * i, g = q >> 2;
     s_act[4 * ((g & 3) * kPcs + (g >> 2)) + (q & 3)] = d;
   }
   __syncthreads();
@@ -522,14 +541,14 @@ __global__ __launch_bounds__(256) void ternary_gemv_norm_vec_kernel(TernaryGemvG
   if (j == 0 && row < m) out[row] = (float)acc * cs;
 }
 
-template <int LPR>
+template <int LPR, int T>
 hipError_t launch_norm_vec(const TernaryGemvGroupArgs &a, const GemvNormArgs &p, int wgs, hipStream_t s) {
-  const dim3 grid(wgs), block(256);
-  const int nq = (a.in_features + 1023) / 1024;
-  if (nq <= 3) ternary_gemv_norm_vec_kernel<3, LPR><<<grid, block, 0, s>>>(a, p);
-  else if (nq <= 4) ternary_gemv_norm_vec_kernel<4, LPR><<<grid, block, 0, s>>>(a, p);
-  else if (nq <= 7) ternary_gemv_norm_vec_kernel<7, LPR><<<grid, block, 0, s>>>(a, p);
-  else ternary_gemv_norm_vec_kernel<8, LPR><<<grid, block, 0, s>>>(a, p);
+  const dim3 grid(wgs), block(T);
+  const int nq = (a.in_features + 4 * T - 1) / (4 * T);
+  if (nq * T <= 768) ternary_gemv_norm_vec_kernel<(768 + T - 1) / T, LPR, T><<<grid, block, 0, s>>>(a, p);
+  else if (nq * T <= 1024) ternary_gemv_norm_vec_kernel<1024 / T, LPR, T><<<grid, block, 0, s>>>(a, p);
+  else if (nq * T <= 1792) ternary_gemv_norm_vec_kernel<(1792 + T - 1) / T, LPR, T><<<grid, block, 0, s>>>(a, p);
+  else ternary_gemv_norm_vec_kernel<2048 / T, LPR, T><<<grid, block, 0, s>>>(a, p);
   return hipGetLastError();
 }
 
@@ -542,9 +561,11 @@ hipError_t launch_ternary_gemv_norm(const TernaryGemvGroupArgs &a, const GemvNor
   if (a.in_features > kNormK) return hipErrorInvalidValue;
   if (vec) {
     switch (p.rows) {
-      case 16: return launch_norm_vec<16>(a, p, wgs, s);
-      case 32: return launch_norm_vec<8>(a, p, wgs, s);
-      case 64: return launch_norm_vec<4>(a, p, wgs, s);
+      case 16:
+        return a.in_features > 4096 ? launch_norm_vec<32, 512>(a, p, wgs, s)
+                                    : launch_norm_vec<16, 256>(a, p, wgs, s);
+      case 32: return launch_norm_vec<8, 256>(a, p, wgs, s);
+      case 64: return launch_norm_vec<8, 512>(a, p, wgs, s);
       default: return hipErrorInvalidValue;
     }
   }

@@ -166,3 +166,41 @@ def test_norm_quant_fused(backend, mode, n, alias):
     diff = host(q).astype(int) - q_ref.astype(int)
     assert np.all(np.abs(diff) <= 1) and np.count_nonzero(diff) <= max(2, n // 200)
     assert abs(float(host(aa)[0]) - s_ref * 127.0) <= 1e-5 * s_ref * 127.0
+
+
+# K at the ends of the per-thread quad counts (1024, 3072, 4096, 7168, 8192 and
+# one weight piece more), rows that give 16, 32 and 64 rows per workgroup, and
+# rows that leave the last one partly filled; K not a multiple of 64: the scalar form
+@pytest.mark.parametrize("k,rows,mode", [(64, (5,), 0), (1024, (40, 7), 1), (1088, (2100,), 0), (3072, (4096, 33), 1),
+                                         (3136, (64,), 2), (4096, (130,), 0), (4160, (16,), 1), (6912, (2560,), 2),
+                                         (7168, (77,), 0), (7232, (8300,), 2), (8192, (31, 9000), 1), (2560, (6912, 6912), 1),
+                                         (100, (50,), 1), (4200, (20,), 2)])
+def test_gemv_norm_group(backend, k, rows, mode):
+    """The norm-fused projection against 64 bits: the residual sum exact; the int8
+    activations within the half-way cases (0.5 % of them off by one)."""
+    case(f"norm-fused gemv K {k} rows {rows} mode {mode}")
+    import torch
+
+    rng = np.random.default_rng(k + sum(rows) + mode)
+    a, b = (rng.standard_normal(k).astype(f32) for _ in range(2))
+    g = rng.uniform(0.8, 1.2, k).astype(f32)
+    mats = [rng.integers(-1, 2, size=(m, k)).astype(np.int8) for m in rows]
+    d = [dev(oracle.pack_rows(m)) for m in mats]
+    outs = [torch.full((m,), float("nan"), device="cuda") for m in rows]
+    scales = [0.05 + 0.01 * i for i in range(len(rows))]
+    h_out = torch.zeros(k, device="cuda") if mode == 1 else None
+    backend.dev_ternary_gemv_norm_group(d, scales, mode, dev(a), dev(b) if mode else None, dev(g), 1e-5, h_out,
+                                        outs, list(rows), k)
+    x = a if mode == 0 else a + b if mode == 1 else np.maximum(a, f32(0)) ** 2 * b
+    if mode == 1:
+        np.testing.assert_array_equal(host(h_out), x)
+    x = x.astype(np.float64)
+    y = x / np.sqrt((x * x).mean() + 1e-5) * g
+    mx = np.abs(y).max()
+    t = y * 127.0 / mx
+    q = np.trunc(t + np.copysign(0.5, t))
+    for w, out, s in zip(mats, outs, scales):
+        acc = host(out).astype(np.float64) / (np.float64(f32(s)) * mx / 127.0)
+        want = w.astype(np.float64) @ q
+        # an fp32 rounding or two of each factor, and the half-way cases
+        assert np.all(np.abs(acc - want) <= 2 + 0.005 * k + 1e-6 * np.abs(want))
