@@ -534,9 +534,10 @@ PrefillChoice plan_prefill_chunk(int n_tokens, int start_pos, int n_kv, int n_cu
   return best;
 }
 
-// Runs of a split launch.  A unit costs its key tiles plus kUnitCost (queries
-// loaded, output or state stored), and a run ends where that cost passes its
-// share; a boundary that would leave fewer than two tiles of a unit on one
+// Runs of a split launch.  A unit costs its key tiles plus a few more (queries
+// loaded, output or state stored, a merge: 6 to 10 us where a tile takes 2.6
+// beside another workgroup's; in short runs most of it overlaps the other's
+// start), and a run ends where that cost passes its share; a boundary that would leave fewer than two tiles of a unit on one
 // side moves to the unit's end there.  With few units every run boundary adds
 // a state that the unit's last workgroup reads alone: for nk tiles in runs
 // of L that is L tile times and nk / L states, kStateCost tiles each, so runs
@@ -544,10 +545,10 @@ PrefillChoice plan_prefill_chunk(int n_tokens, int start_pos, int n_kv, int n_cu
 // one with issue priority (even runs) takes kEven of their share.  The
 // constants are the best of a sweep over 15 shapes (16 to 4000 tokens, 0 to
 // 4000 cached rows, 20/5 heads, MI355X): a unit cost of 2 / 3 / 4 / 6 tiles
-// takes 46 / 42 / 43 / 46 us at 1024 tokens and 281 / 267 / 259 / 259 us at
-// 4000, a shortest run of 1 / 2 / 3 tiles 33 / 29 / 30 us at 512.
+// takes 46 / 42 / 43 / 46 us at 1024 tokens (5 tiles a run), 60 us or more but
+// for 3 and 4 at 1500, 102 / 94 / 95 / 90 us at 2048 (20) and 281 / 267 / 259 /
+// 259 us at 4000, a shortest run of 1 / 2 / 3 tiles 33 / 29 / 30 us at 512.
 bool plan_prefill_runs(PrefillRunsArgs &a, int group, int n_cu, long long max_slots) {
-  constexpr int kUnitCost = 3;
   constexpr double kStateCost = 0.35, kEven = 0.54, kShortest = 2.0;
   const int uq = split_unit(group), per_cu = split_waves(group) == 4 ? 2 : 1;
   const double even = per_cu == 2 ? 2.0 * kEven : 1.0;
@@ -560,8 +561,10 @@ bool plan_prefill_runs(PrefillRunsArgs &a, int group, int n_cu, long long max_sl
   const int nk_max = nk(a.n_units - 1);
   if (nk_max > 65535) return false;
   long long total = 0;
-  for (int u = 0; u < a.n_units; ++u) total += nk(u) + kUnitCost;
-  const double shortest = std::max(kShortest, std::sqrt(nk_max * kStateCost)) + kUnitCost;
+  for (int u = 0; u < a.n_units; ++u) total += nk(u);
+  const int unit_cost = total > 12 * std::min<long long>(per_cu * n_cu / a.n_kv, kMaxPrefillRuns) ? 6 : 3;
+  total += (long long)unit_cost * a.n_units;
+  const double shortest = std::max(kShortest, std::sqrt(nk_max * kStateCost)) + unit_cost;
   long long P = std::min<long long>(std::max(1, per_cu * n_cu / a.n_kv), kMaxPrefillRuns);
   P = std::max(1LL, std::min(P, (long long)(total / shortest)));
   struct Cut {
@@ -577,9 +580,9 @@ bool plan_prefill_runs(PrefillRunsArgs &a, int group, int n_cu, long long max_sl
     int u = 0;
     for (long long r = 1; r < P; ++r) {
       const long long x = (long long)(total * (double)((r / 2) * 2 + (r & 1) * even) / P);
-      while (u < a.n_units && x >= off + nk(u) + kUnitCost) off += nk(u++) + kUnitCost;
+      while (u < a.n_units && x >= off + nk(u) + unit_cost) off += nk(u++) + unit_cost;
       if (u >= a.n_units) break;
-      Cut c{u, (int)std::max(0LL, x - off - kUnitCost)};
+      Cut c{u, (int)std::max(0LL, x - off - unit_cost)};
       if (c.kt < 2) c.kt = 0;
       if (c.kt > nk(u) - 2 && c.kt > 0) c = Cut{u + 1, 0};
       if (c.u >= a.n_units) break;
