@@ -225,12 +225,11 @@ __global__ __launch_bounds__(256) void ternary_gemv_group_kernel(TernaryGemvGrou
 // forms x from f32 inputs (a | a + b | max(a,0)^2 * b), reduces sum(x^2) and
 // max|y| with the same tree, and so derives the same int8 activations and
 // the same scale as norm_quant_kernel would; the int8 vector never leaves
-// LDS.  The workgroup issues the (cache-resident) activation loads first and
-// its weight loads right after, so the prologue runs under the weights'
-// latency.  K <= 4096 NG (one LDS pass; NG = 1 or 2 16-activation groups
-// per thread, the smallest that holds K: at K <= 4096 the kernel needs 74
-// VGPRs and 6 workgroups fit a CU, with two groups 142 and 3);
-// workgroup 0 writes h_out (mode residual), which must not alias a or b.
+// LDS.  The aligned kernel below issues the (cache-resident) activation loads
+// first and its weight loads right after, so the prologue runs under the
+// weights' latency; the one here takes unaligned rows and vectors and any K <=
+// 4096 NG (NG = 1 or 2 16-activation groups per thread), element by element.
+// Workgroup 0 writes h_out (mode residual), which must not alias a or b.
 // A workgroup owns 256 / LPR rows, LPR lanes per row: every workgroup reads
 // the whole of a (and b) and gamma, so a launch with many rows takes 32 or
 // 64 rows per workgroup to read those vectors fewer times.
@@ -611,7 +610,8 @@ hipError_t launch_ternary_gemv(const TernaryGemvArgs &a, bool vec, hipStream_t s
 // staged in LDS once per pass of 4096 values, is reused over 320 KB of
 // weights; the next block's pieces are loaded while the current block is
 // multiplied.  fp32 products and sums (any order; the reference's AVX2 lane
-// order is not reproduced, results agree to rounding).
+// order is not reproduced, results agree to rounding).  For unaligned weights
+// and K > kLmMaxK; the aligned form is lm_head_mfma_kernel.
 // ---------------------------------------------------------------------------
 namespace bnr {
 namespace {

@@ -534,20 +534,21 @@ PrefillChoice plan_prefill_chunk(int n_tokens, int start_pos, int n_kv, int n_cu
   return best;
 }
 
-// Runs of a split launch.  A unit costs its key tiles plus a few more (queries
-// loaded, output or state stored, a merge: 6 to 10 us where a tile takes 2.6
-// beside another workgroup's; in short runs most of it overlaps the other's
-// start), and a run ends where that cost passes its share; a boundary that would leave fewer than two tiles of a unit on one
-// side moves to the unit's end there.  With few units every run boundary adds
-// a state that the unit's last workgroup reads alone: for nk tiles in runs
-// of L that is L tile times and nk / L states, kStateCost tiles each, so runs
-// are no shorter than sqrt(nk kStateCost).  Of two workgroups on a CU the
-// one with issue priority (even runs) takes kEven of their share.  The
-// constants are the best of a sweep over 15 shapes (16 to 4000 tokens, 0 to
-// 4000 cached rows, 20/5 heads, MI355X): a unit cost of 2 / 3 / 4 / 6 tiles
-// takes 46 / 42 / 43 / 46 us at 1024 tokens (5 tiles a run), 60 us or more but
-// for 3 and 4 at 1500, 102 / 94 / 95 / 90 us at 2048 (20) and 281 / 267 / 259 /
-// 259 us at 4000, a shortest run of 1 / 2 / 3 tiles 33 / 29 / 30 us at 512.
+// Runs of a split launch.  A unit costs its key tiles plus unit_cost more
+// (queries loaded, output or state stored, a merge: 6 to 10 us where a tile
+// takes 2.6 beside another workgroup's; in short runs most of it overlaps the
+// other's start), and a run ends where that cost passes its share; a boundary
+// that would leave fewer than two tiles of a unit on one side moves to the
+// unit's end there.  With few units every run boundary adds a state that the
+// unit's last workgroup reads alone: for nk tiles in runs of L that is L tile
+// times and nk / L states, kStateCost tiles each, so runs are no shorter than
+// sqrt(nk kStateCost).  Of two workgroups on a CU the one with issue priority
+// (even runs) takes kEven of their share.  The constants are the best of a
+// sweep over 15 shapes (16 to 4000 tokens, 0 to 4000 cached rows, 20/5 heads,
+// MI355X, RoPE + append + attention): a unit cost of 2 / 3 / 4 / 6 tiles takes
+// 46 / 42 / 43 / 46 us at 1024 tokens (5 tiles a run), 64 / 60 / 60 / 60 us at
+// 1500 (11), 102 / 94 / 95 / 90 us at 2048 (20) and 281 / 267 / 259 / 259 us at
+// 4000 (78); a shortest run of 1 / 2 / 3 tiles 33 / 29 / 30 us at 512.
 bool plan_prefill_runs(PrefillRunsArgs &a, int group, int n_cu, long long max_slots) {
   constexpr double kStateCost = 0.35, kEven = 0.54, kShortest = 2.0;
   const int uq = split_unit(group), per_cu = split_waves(group) == 4 ? 2 : 1;
