@@ -1763,7 +1763,7 @@ long long split_slots(const bnr_ctx *c, long long cap, int n_kv, int group) {
   const int per_cu = group >= 8 ? 1 : 2;
   const long long items = std::max(prefill_item_budget(cap, n_kv), 2LL * c->n_cu * per_cu);
   return (items * group * 66 * 64 - split_tile_floats(cap, n_kv)) /
-         ((long long)split_waves(group) * 66 * 64 * n_kv);
+         ((long long)split_waves(group) * kSplitStateFloats * n_kv);
 }
 
 // Whether a prefill of a tiled shape runs as a split launch: nothing else is
@@ -1786,7 +1786,7 @@ bool prefill_split_plan(const bnr_ctx *c, size_t n_tokens, size_t start_pos, siz
                         size_t n_heads, size_t n_kv, PrefillRunsArgs &a) {
   const int group = (int)(n_heads / n_kv);
   const long long slots = split_slots(c, (long long)cap, (int)n_kv, group);
-  if (slots * split_waves(group) * 66 * 64 * (long long)n_kv < split_tile_floats((long long)cap, (int)n_kv))
+  if (slots * split_waves(group) * kSplitStateFloats * (long long)n_kv < split_tile_floats((long long)cap, (int)n_kv))
     return false;
   a.n_tokens = (int)n_tokens;
   a.start_pos = (int)start_pos;

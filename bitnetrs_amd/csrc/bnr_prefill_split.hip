@@ -111,13 +111,21 @@ constexpr int kSplitFp32 = 0x100, kSplitZero = 0x200;
 // From the largest and the smallest nonzero row maximum (bits; ~0: no
 // nonzero row): fp32 for infinities and NaN, for rows whose largest value is
 // below 2^-15 of the tile's (an fp16 subnormal would cut them off above
-// 2^-24 of that value) and for tiles whose scale would pass 2^126.
+// 2^-24 of that value) and for tiles whose scale would pass 2^126.  A marked
+// tile's exponent says how large its values are: O takes it for its own.
 __device__ __forceinline__ int tile_word(unsigned mx, unsigned mn) {
   constexpr unsigned kSplitRange = 15;
   if (mx == 0) return 128 | kSplitZero;
   const unsigned e = mx >> 23;
-  if (e == 255 || e < 15 || (mn >> 23) + kSplitRange < e) return 128 | kSplitFp32;
-  return scale_exp(mx) + 128;
+  const int word = scale_exp(mx) + 128;
+  return e == 255 || e < 15 || (mn >> 23) + kSplitRange < e ? word | kSplitFp32 : word;
+}
+// The scale exponent that a V tile asks of O.  A marked tile's values are not
+// scaled: the limits keep its weights, 2^(15 + exponent) at most, and their
+// products with the values inside fp32.
+__device__ __forceinline__ int v_exp(int word) {
+  const int e = (word & 255) - 128;
+  return (word & kSplitFp32) ? min(max(e, -50), 100) : e;
 }
 
 // One 32-key tile of one kv head per workgroup (blockIdx.x < n_kv * n_tiles,
@@ -333,7 +341,9 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
 // range with its low half normal down to 2^-14 of the reference.  ev is the V
 // tile's scale exponent, E the one O carries: O moves to another tile's scale
 // only when that tile's V is larger than E allows (ev < E) or 2^8 smaller, so
-// P gives up at most 8 of those 14 bits.
+// P gives up at most 8 of those 14 bits.  The output is (O / l) 2^-E: 2^E is
+// undone last (O alone, with 2^11 and the sum of the weights in it, would pass
+// fp32's largest value where the output does not).
 // ---------------------------------------------------------------------------
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Wpass-failed"
@@ -531,8 +541,7 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     mb = max_half_swap(mb) * c;
     // O moves to another reference (some query's maximum passed its own by
     // kLazy) or to this tile's scale (uniform over the wave): rare.
-    int ev = (wv & kSplitFp32) ? 0 : (wv & 255) - 128;
-    if (wv & kSplitZero) ev = E;
+    const int ev = (wv & kSplitZero) ? E : v_exp(wv);
     if (__ballot(mb > m + kLazy) != 0 || ev < E || ev > E + kScaleSlack) {
       int en = E;
       if (ev < E || ev > E + kScaleSlack) {
@@ -565,7 +574,11 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     split8p(p, 8, ph, pl);
     mm_o(A, 0, ph, pl);
     mm_o(B, 2, ph, pl);
-    if (wv & kSplitFp32) sp_fp32_pv(a, h, kt, p, O);
+    if (wv & kSplitFp32) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) p[r] = ldexpf(p[r], ev);
+      sp_fp32_pv(a, h, kt, p, O);
+    }
   };
 
   // Queries of the unit's block: lane's dims 16 s + 8 hl + i of query q0 + col
@@ -604,27 +617,23 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     // key at all (p = 0 for it throughout, and no -inf - -inf).
     m = -1e30f;
     l = 0.f;
-    E = (word & (kSplitFp32 | kSplitZero)) ? 0 : (word & 255) - 128;
+    E = (word & kSplitZero) ? 0 : v_exp(word);
     e_min = E;
   };
 
   // End of a piece: one of several stores its state and takes a ticket; the
   // unit's last to finish adds the others to its registers and, like a whole
   // unit, writes the output.  State of a wave: float4 k (components 4k ..
-  // 4k+3 of O, 16 db + r) of lane l at float (k * 64 + l) * 4, then (m, l) at
-  // 64 * 64 + 2 l.
+  // 4k+3 of O, 16 db + r) of lane l at float (k * 64 + l) * 4, then (m, l, E)
+  // at 64 * 64 + 4 l.
   auto finish = [&](int nch, int ch, int base) {
     // lane values hidden from the compiler, which would otherwise form the
     // addresses below ahead of the tile loop and keep them in registers
     int lane = tid & 63;
     asm volatile("" : "+v"(lane));
     const int hl = lane >> 5, col = lane & 31;
-#pragma unroll
-    for (int db = 0; db < 4; ++db)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) O[db][r] = ldexpf(O[db][r], -E);
     auto state = [&](int c) {
-      return agent_buf(a.ws + (((long long)h * a.n_slots + base + c) * W + wave) * 66 * 64);
+      return agent_buf(a.ws + (((long long)h * a.n_slots + base + c) * W + wave) * kSplitStateFloats);
     };
     if (nch > 1) {
       const __amdgpu_buffer_rsrc_t mine = state(ch);
@@ -633,7 +642,7 @@ void prefill_split_kernel(PrefillRunsArgs a) {
         st4_agent(mine, lane * 16, 1024 * k,
                   make_float4(O[k >> 2][4 * (k & 3)], O[k >> 2][4 * (k & 3) + 1],
                               O[k >> 2][4 * (k & 3) + 2], O[k >> 2][4 * (k & 3) + 3]));
-      st2_agent(mine, 64 * 64 * 4 + 8 * lane, m, l);
+      st4_agent(mine, 64 * 64 * 4 + 16 * lane, make_float4(m, l, (float)E, 0.f));
       __builtin_amdgcn_s_waitcnt(0);  // this wave's state has been stored
       __syncthreads();
       unsigned *ctr = a.counters + ((long long)h * a.n_units + u) * kCounterStride;
@@ -648,20 +657,23 @@ void prefill_split_kernel(PrefillRunsArgs a) {
       if (!last) return;  // s_last is written again only past the next tile's barrier
       if (tid == 0) __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       struct State {
-        float4 o[16];
-        float2 ml;
+        float4 o[16], mle;
       };
       auto load = [&](State &x, int c) {
         const __amdgpu_buffer_rsrc_t src = state(c);
 #pragma unroll
         for (int k = 0; k < 16; ++k) x.o[k] = ld4_agent(src, lane * 16, 1024 * k);
-        x.ml = ld2_agent(src, 64 * 64 * 4 + 8 * lane);
+        x.mle = ld4_agent(src, 64 * 64 * 4 + 16 * lane);
       };
       auto add = [&](const State &x) {
-        const float mn = fmaxf(m, x.ml.x);
-        const float wa = fast_exp2(m - mn), wb = fast_exp2(x.ml.x - mn);
-        l = l * wa + x.ml.y * wb;
+        const float mn = fmaxf(m, x.mle.x);
+        const int xe = (int)x.mle.z, en = min(E, xe);
+        float wa = fast_exp2(m - mn), wb = fast_exp2(x.mle.x - mn);
+        l = l * wa + x.mle.y * wb;
         m = mn;
+        wa = ldexpf(wa, en - E);
+        wb = ldexpf(wb, en - xe);
+        E = en;
 #pragma unroll
         for (int k = 0; k < 16; ++k) {
           floatx16 &o = O[k >> 2];
@@ -687,7 +699,8 @@ void prefill_split_kernel(PrefillRunsArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         st4(op + 32 * (r >> 2) + 4 * (r & 3),
-            make_float4(O[0][r] * inv, O[1][r] * inv, O[2][r] * inv, O[3][r] * inv));
+            make_float4(ldexpf(O[0][r] * inv, -E), ldexpf(O[1][r] * inv, -E),
+                        ldexpf(O[2][r] * inv, -E), ldexpf(O[3][r] * inv, -E)));
     }
     SP_STAMP(kPfStored);
   };

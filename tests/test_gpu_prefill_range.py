@@ -1,0 +1,86 @@
+"""Split prefill over the range of fp32: finite inputs whose magnitudes lie far
+apart -- between the values of a row, between head dims, between rows and
+between tiles -- against 64 bits, each output column and each query row by
+itself, beside the fp32 launches on the same inputs."""
+import sys
+
+import pytest
+
+from common import D
+
+pytestmark = pytest.mark.gpu
+
+HQ, HKV = 8, 2
+
+
+def case(msg):
+    print(f"[case] {msg}", flush=True)
+    sys.stdout.flush()
+
+
+def attend(monkeypatch, split, q, kc, vc, start):
+    import torch
+
+    import bitnetrs_amd
+
+    monkeypatch.setenv("BNR_PREFILL_SPLIT", str(split))
+    n, n_heads, n_kv, cap = q.shape[0], q.shape[1] // D, kc.shape[0], kc.shape[1]
+    gpu = bitnetrs_amd.HipBackend(0)
+    out = torch.zeros_like(q)
+    gpu.dev_prefill_attention(q, kc, vc, cap, out, n, start, n_heads, n_kv, D)
+    torch.cuda.synchronize()
+    gpu.close()
+    return out
+
+
+def attend64(q, kc, vc, start):
+    """Rows of q [n, heads * D] over cache rows 0 .. start + i in 64 bits."""
+    import torch
+
+    n, n_heads, n_kv, rows = q.shape[0], q.shape[1] // D, kc.shape[0], start + q.shape[0]
+    hidden = (torch.arange(rows)[None, :] > start + torch.arange(n)[:, None]).to(q.device)
+    out = torch.empty(n, n_heads, D, dtype=torch.float64, device=q.device)
+    q = q.double().reshape(n, n_heads, D)
+    for h in range(n_heads):
+        k, v = kc[h * n_kv // n_heads, :rows].double(), vc[h * n_kv // n_heads, :rows].double()
+        s = (q[:, h] @ k.t().contiguous()) / D ** 0.5
+        out[:, h] = torch.softmax(s.masked_fill(hidden, float("-inf")), 1) @ v
+    return out
+
+
+def normal(n, start, seed, n_heads=HQ, n_kv=HKV):
+    import torch
+
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    cap = start + n
+    return (torch.randn(n, n_heads * D, device="cuda", generator=g),
+            torch.randn(n_kv, cap, D, device="cuda", generator=g),
+            torch.randn(n_kv, cap, D, device="cuda", generator=g))
+
+
+def worst(out, ref, by):
+    """The largest relative error (2-norm) of any (head, column) or (row, head)."""
+    out = out.double().reshape(ref.shape)
+    assert bool(out.isfinite().all()), "not finite"
+    dim = 0 if by == "column" else 2
+    scale = ref.abs().amax().item() or 1.0  # norms of values near fp32's ends
+    d, r = ((out - ref) / scale).norm(dim=dim), (ref / scale).norm(dim=dim)
+    return (d / r.clamp_min(1e-300)).max().item()
+
+
+# a constant V: the output is that value, whatever is added up on the way
+@pytest.mark.parametrize("c", [1e30, 1e33, 1e36, 3e38])
+@pytest.mark.parametrize("marked", [False, True])
+def test_large_v(monkeypatch, c, marked):
+    case(f"split prefill, V of {c}, marked tiles {marked}")
+    import torch
+
+    n, start = 1024, 1024
+    q, kc, vc = normal(n, start, 11)
+    q *= 0.1  # weights spread over all keys
+    vc.fill_(c)
+    if marked:
+        vc[:, ::32] = c * 2.0 ** -20  # rows far apart in every tile
+    ref = attend64(q, kc, vc, start)
+    out = attend(monkeypatch, 1, q, kc, vc, start)
+    assert worst(out, ref, "column") <= 2.0 ** -20 and worst(out, ref, "row") <= 2.0 ** -20
