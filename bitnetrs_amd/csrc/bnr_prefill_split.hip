@@ -69,6 +69,25 @@ __device__ __forceinline__ void split8(const float (&x)[8], half8 &h, half8 &l) 
   }
 }
 
+// p[r] .. p[r + 7] times f (a power of two) -> h and l: l is what h leaves of
+// the product, formed and rounded in one instruction (v_fma_mixlo, _mixhi).
+// The empty asm keeps the compiler from converting the products a second time.
+__device__ __forceinline__ void split8f(const float (&p)[16], int r, float f, half8 &h, half8 &l) {
+  typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+  typedef float float2_t __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int i = 0; i < 8; i += 2) {
+    const float x = p[r + i], y = p[r + i + 1];
+    unsigned w = __builtin_bit_cast(unsigned, __builtin_convertvector((float2_t{x * f, y * f}), half2_t));
+    asm("" : "+v"(w));
+    const half2_t a = __builtin_bit_cast(half2_t, w);
+    h[i] = a.x;
+    h[i + 1] = a.y;
+    l[i] = (_Float16)fmaf(x, f, -(float)a.x);
+    l[i + 1] = (_Float16)fmaf(y, f, -(float)a.y);
+  }
+}
+
 __device__ __forceinline__ unsigned abs_bits(float x) {
   return __builtin_bit_cast(unsigned, x) & 0x7fffffffu;
 }
@@ -335,21 +354,23 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
 // fp32 products.  One 8-wave workgroup of 64 queries per CU (half the
 // operand traffic, one barrier per 64 keys) took 47, 93 and 48 us.
 //
-// p = exp2(S c + 11 + (E - ev) - m): c undoes the scales of K and q and
-// applies log2(e) / sqrt(d); m is a lazily moved reference (it follows a
-// query's maximum once that passes it by 4), and 2^11 puts p <= 2^15 in fp16
-// range with its low half normal down to 2^-14 of the reference.  ev is the V
-// tile's scale exponent, E the one O carries: O moves to another tile's scale
-// only when that tile's V is larger than E allows (ev < E) or 2^8 smaller, so
-// P gives up at most 8 of those 14 bits.  The output is (O / l) 2^-E: 2^E is
+// p = exp2(S c - m): c undoes the scales of K and q and applies log2(e) /
+// sqrt(d); m is a lazily moved reference (it follows a query's maximum once
+// that passes it by 4).  The operand is p 2^(11 + E - ev): 2^11 puts it below
+// 2^15 in fp16 range with its low half normal down to 2^-14 of the reference.
+// (It is a factor, not part of the exponential's argument: that would be
+// rounded near 11 where it is rounded near 0.)  ev is the V tile's scale
+// exponent, E the one O carries: O moves to another tile's scale only when
+// that tile's V is larger than E allows (ev < E) or 2^8 smaller, so P gives up
+// at most 8 of those 14 bits.  The output is (O / l) 2^-(E + 11): the scale is
 // undone last (O alone, with 2^11 and the sum of the weights in it, would pass
 // fp32's largest value where the output does not).
 // ---------------------------------------------------------------------------
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Wpass-failed"
 
-constexpr float kPShift = 11.0f, kLazy = 4.0f;
-constexpr int kScaleSlack = 8, kScaleSpan = 60;
+constexpr float kLazy = 4.0f;
+constexpr int kPShift = 11, kScaleSlack = 8, kScaleSpan = 60;
 
 __device__ __forceinline__ float max_half_swap(float v) {  // max over lanes l, l ^ 32
   const unsigned u = __builtin_bit_cast(unsigned, v);
@@ -504,10 +525,6 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     mm(x[0], ph, O[db]);
     mm(x[2], ph, O[db + 1]);
   };
-  auto split8p = [](const float (&p)[16], int r, half8 &h8, half8 &l8) {
-    const float y[8] = {p[r], p[r + 1], p[r + 2], p[r + 3], p[r + 4], p[r + 5], p[r + 6], p[r + 7]};
-    split8(y, h8, l8);
-  };
 
   // The products of one tile (operands at dk, words wk and wv).
   auto step = [&](const float *dk, int kt, int wk, int wv) {
@@ -556,27 +573,27 @@ void prefill_split_kernel(PrefillRunsArgs a) {
       m = mn;
       E = en;
     }
-    const float add = kPShift + (float)(E - ev) - m;
     float p[16], ls = 0.f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      p[r] = fast_exp2(fmaf(S[r], c, add));
+      p[r] = fast_exp2(fmaf(S[r], c, -m));
       ls += p[r];
     }
-    l = fmaf(ls, ldexpf(1.0f, ev - E), l);
+    l += ls;
+    const float f = ldexpf(1.0f, kPShift + E - ev);
     half8 ph, pl;
-    split8p(p, 0, ph, pl);
+    split8f(p, 0, f, ph, pl);
     rd(B, dv, 4);
     mm_o(A, 0, ph, pl);
     rd(A, dv, 8);
     mm_o(B, 2, ph, pl);
     rd(B, dv, 12);
-    split8p(p, 8, ph, pl);
+    split8f(p, 8, f, ph, pl);
     mm_o(A, 0, ph, pl);
     mm_o(B, 2, ph, pl);
     if (wv & kSplitFp32) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) p[r] = ldexpf(p[r], ev);
+      for (int r = 0; r < 16; ++r) p[r] = ldexpf(p[r], kPShift + E);
       sp_fp32_pv(a, h, kt, p, O);
     }
   };
@@ -699,8 +716,8 @@ void prefill_split_kernel(PrefillRunsArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         st4(op + 32 * (r >> 2) + 4 * (r & 3),
-            make_float4(ldexpf(O[0][r] * inv, -E), ldexpf(O[1][r] * inv, -E),
-                        ldexpf(O[2][r] * inv, -E), ldexpf(O[3][r] * inv, -E)));
+            make_float4(ldexpf(O[0][r] * inv, -(E + kPShift)), ldexpf(O[1][r] * inv, -(E + kPShift)),
+                        ldexpf(O[2][r] * inv, -(E + kPShift)), ldexpf(O[3][r] * inv, -(E + kPShift))));
     }
     SP_STAMP(kPfStored);
   };
