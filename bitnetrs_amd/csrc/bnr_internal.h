@@ -553,7 +553,7 @@ hipError_t launch_prefill_split_kv(const PrefillSplitArgs &p, hipStream_t s);
 // nch - 1 of the kv head, and the last to finish merges them.
 constexpr int split_waves(int group) { return group > 4 ? 8 : 4; }
 constexpr int split_unit(int group) { return 32 * split_waves(group) / group; }
-constexpr int kSplitStateFloats = 68 * 64;  // a wave's state: O, and (m, l, E, -) of every lane
+constexpr int kSplitStateFloats = 68 * 64;  // a wave's state: O, and (m, l, g, -) of every lane
 constexpr int kMaxPrefillRuns = 256;
 struct PrefillRunsArgs {
   const float *q;                  // [n_tokens][n_heads][128], rotated

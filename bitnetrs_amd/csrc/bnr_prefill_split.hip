@@ -355,22 +355,28 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
 // operand traffic, one barrier per 64 keys) took 47, 93 and 48 us.
 //
 // p = exp2(S c - m): c undoes the scales of K and q and applies log2(e) /
-// sqrt(d); m is a lazily moved reference (it follows a query's maximum once
-// that passes it by 4).  The operand is p 2^(11 + E - ev): 2^11 puts it below
-// 2^15 in fp16 range with its low half normal down to 2^-14 of the reference.
-// (It is a factor, not part of the exponential's argument: that would be
-// rounded near 11 where it is rounded near 0.)  ev is the V tile's scale
-// exponent, E the one O carries: O moves to another tile's scale only when
-// that tile's V is larger than E allows (ev < E) or 2^8 smaller, so P gives up
-// at most 8 of those 14 bits.  The output is (O / l) 2^-(E + 11): the scale is
-// undone last (O alone, with 2^11 and the sum of the weights in it, would pass
-// fp32's largest value where the output does not).
+// sqrt(d); m is a lazily moved whole number above or near the query's largest
+// S c.  (The power of two below is a factor, not part of the exponential's
+// argument: that would be rounded near 11 where it is rounded near 0.)
+//
+// O holds sum(p V) 2^g, g a whole number per query, and the operand is p
+// 2^(g - ev) for a V tile of scale exponent ev.  g stays while the tile's
+// largest operand lies between 2^1 (what fp16's subnormals cut off is then 2^-26
+// of it) and 2^15, else it is moved to 2^8, and O with it.  Weights and
+// V so far below what O holds that it would overflow (kScaleSpan), and weights
+// near fp32's end, take fp32 products for that tile.  The output is (O / l)
+// 2^-g in that order: O alone, with the sum of the weights and a power of two in
+// it, would pass fp32's largest value where the output does not.
 // ---------------------------------------------------------------------------
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Wpass-failed"
 
-constexpr float kLazy = 4.0f;
-constexpr int kPShift = 11, kScaleSlack = 8, kScaleSpan = 60;
+constexpr float kLazy = 4.0f, kNoRef = -3.4028234e38f, kLeastP = -126.0f, kPHalf = 7.0f;
+constexpr int kPMid = 8;           // operands: the tile's largest is 2^8, in 2^(8 -+ 7)
+constexpr int kScaleSpan = 72;     // sum(p V) 2^g <= 2^23 times the keys, and 2^72 more once g follows V down
+constexpr int kNoScale = 1 << 28;   // O holds nothing yet
+constexpr int kMaxFactor = 112;     // of 2^(g - ev), a float
+constexpr int kMaxShift = 4096;     // more than any O keeps
 
 __device__ __forceinline__ float max_half_swap(float v) {  // max over lanes l, l ^ 32
   const unsigned u = __builtin_bit_cast(unsigned, v);
@@ -406,11 +412,13 @@ __device__ __forceinline__ floatx16 sp_fp32_s(const PrefillRunsArgs &a, int h, i
 __device__ __forceinline__ void sp_fp32_pv(const PrefillRunsArgs &a, int h, int kt,
                                            const float (&p)[16], floatx16 (&O)[4]) {
   const int lane = threadIdx.x & 63, hl = lane >> 5, col = lane & 31;
-  const float *vp = a.v_cache + h * a.kv_stride + 4 * col;
+  const float *vp = a.v_cache + h * a.kv_stride + (long long)kt * 32 * kHeadDim;  // uniform
+  const int last = a.start_pos + a.n_tokens - 1 - kt * 32;
 #pragma unroll
   for (int s = 0; s < 16; ++s) {
-    const int row = min(kt * 32 + 8 * (s >> 2) + 4 * hl + (s & 3), a.start_pos + a.n_tokens - 1);
-    const float4 vv = ld4(vp + (long long)row * kHeadDim);
+    if ((s & 3) == 0) __builtin_amdgcn_sched_barrier(0);  // the loads of four steps at a time
+    const int row = min(8 * (s >> 2) + 4 * hl + (s & 3), last);
+    const float4 vv = ld4(vp + (unsigned)(row * kHeadDim + 4 * col));
     O[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.x, p[s], O[0], 0, 0, 0);
     O[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.y, p[s], O[1], 0, 0, 0);
     O[2] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.z, p[s], O[2], 0, 0, 0);
@@ -495,7 +503,7 @@ void prefill_split_kernel(PrefillRunsArgs a) {
   half8 qh[8], ql[8];
   floatx16 O[4];
   float cq, m, l;
-  int E, e_min, qrow, q0;
+  int g, g_cap, qrow, q0;
   const float *qp;
 
   // Four operands read ahead of the products that use them (two sets of
@@ -555,23 +563,43 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     float mb = S[0];
 #pragma unroll
     for (int r = 1; r < 16; ++r) mb = fmaxf(mb, S[r]);
-    mb = max_half_swap(mb) * c;
-    // O moves to another reference (some query's maximum passed its own by
-    // kLazy) or to this tile's scale (uniform over the wave): rare.
-    const int ev = (wv & kSplitZero) ? E : v_exp(wv);
-    if (__ballot(mb > m + kLazy) != 0 || ev < E || ev > E + kScaleSlack) {
-      int en = E;
-      if (ev < E || ev > E + kScaleSlack) {
-        e_min = min(e_min, ev);
-        en = min(ev, e_min + kScaleSpan);  // no overflow of what O holds
+    mb = max_half_swap(mb);
+    // m or g moves for some query (uniform over the wave): rare.
+    const int ev = v_exp(wv);
+    const bool zero_v = (wv & kSplitZero) != 0;
+    bool fp32_v = (wv & kSplitFp32) != 0;
+    // t: log2 of the tile's largest weight; off: of its largest operand, past
+    // the middle of the range.  One comparison for "t > kLazy, |off| > kPHalf
+    // or a factor too large".
+    float t = fmaf(mb, c, -m);
+    auto off = [&] { return t + (float)(g - ev - kPMid); };
+    const float worst = fmaxf(fmaxf(fabsf(off()), t + (kPHalf - kLazy)), (float)(g - ev - kMaxFactor) + kPHalf);
+    if (zero_v || __ballot(worst > kPHalf) != 0) {
+      if (t > kLazy) {
+        const float mn = ceilf(mb * c);
+        const int up = (int)fminf(mn - m, (float)kMaxShift);
+        l *= fast_exp2(m - mn);
+        g += up;
+        g_cap += up;
+        m = mn;
+        t = fmaf(mb, c, -m);
       }
-      const float mn = mb > m + kLazy ? mb : m;
-      const float alpha = fast_exp2(m - mn), f = ldexpf(alpha, en - E);
-      l *= alpha;
+      if (!zero_v) {
+        // queries that see no key of the tile, or none with a weight, stay
+        const bool has = t >= kLeastP;
+        const int want = kPMid - (int)ceilf(fmaxf(t, kLeastP));
+        if (has) g_cap = min(g_cap, want + (wv & 255) - 128 + kScaleSpan);
+        const bool move = has && (fabsf(off()) > kPHalf || g - ev > kMaxFactor);
+        const int gn = move ? min(min(want, kMaxFactor) + ev, g_cap) : g;
+        if (__ballot(gn != g) != 0) {
 #pragma unroll
-      for (int db = 0; db < 4; ++db) O[db] *= f;
-      m = mn;
-      E = en;
+          for (int db = 0; db < 4; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) O[db][r] = ldexpf(O[db][r], gn - g);
+          g = gn;
+        }
+        fp32_v = fp32_v || __ballot(has && off() < -kPHalf) != 0;
+      }
     }
     float p[16], ls = 0.f;
 #pragma unroll
@@ -580,7 +608,10 @@ void prefill_split_kernel(PrefillRunsArgs a) {
       ls += p[r];
     }
     l += ls;
-    const float f = ldexpf(1.0f, kPShift + E - ev);
+    if (zero_v) return;
+    // fp32 products come after these, whose factor is then 0 (a branch around
+    // them would cost 24 more registers than there are)
+    const float f = fp32_v ? 0.f : ldexpf(1.0f, min(g - ev, kMaxFactor));
     half8 ph, pl;
     split8f(p, 0, f, ph, pl);
     rd(B, dv, 4);
@@ -591,16 +622,16 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     split8f(p, 8, f, ph, pl);
     mm_o(A, 0, ph, pl);
     mm_o(B, 2, ph, pl);
-    if (wv & kSplitFp32) {
+    if (fp32_v) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) p[r] = ldexpf(p[r], kPShift + E);
+      for (int r = 0; r < 16; ++r) p[r] = ldexpf(p[r], g);
       sp_fp32_pv(a, h, kt, p, O);
     }
   };
 
   // Queries of the unit's block: lane's dims 16 s + 8 hl + i of query q0 + col
   // (rows past the end repeat the last and are not stored), as fp16 pairs.
-  auto begin = [&](int word) {
+  auto begin = [&] {
     int lane = tid & 63;
     asm volatile("" : "+v"(lane));
     const int hl = lane >> 5, col = lane & 31;
@@ -632,16 +663,16 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     for (int db = 0; db < 4; ++db) O[db] = floatx16{};
     // m starts finite: in a piece that is not the first, a query may see no
     // key at all (p = 0 for it throughout, and no -inf - -inf).
-    m = -1e30f;
+    m = kNoRef;
     l = 0.f;
-    E = (word & kSplitZero) ? 0 : v_exp(word);
-    e_min = E;
+    g = 0;
+    g_cap = kNoScale;
   };
 
   // End of a piece: one of several stores its state and takes a ticket; the
   // unit's last to finish adds the others to its registers and, like a whole
   // unit, writes the output.  State of a wave: float4 k (components 4k ..
-  // 4k+3 of O, 16 db + r) of lane l at float (k * 64 + l) * 4, then (m, l, E)
+  // 4k+3 of O, 16 db + r) of lane l at float (k * 64 + l) * 4, then (m, l, g)
   // at 64 * 64 + 4 l.
   auto finish = [&](int nch, int ch, int base) {
     // lane values hidden from the compiler, which would otherwise form the
@@ -652,6 +683,7 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     auto state = [&](int c) {
       return agent_buf(a.ws + (((long long)h * a.n_slots + base + c) * W + wave) * kSplitStateFloats);
     };
+    if (g_cap >= kNoScale / 2) g = kMaxShift;  // an empty O asks for no scale in a merge
     if (nch > 1) {
       const __amdgpu_buffer_rsrc_t mine = state(ch);
 #pragma unroll
@@ -659,7 +691,7 @@ void prefill_split_kernel(PrefillRunsArgs a) {
         st4_agent(mine, lane * 16, 1024 * k,
                   make_float4(O[k >> 2][4 * (k & 3)], O[k >> 2][4 * (k & 3) + 1],
                               O[k >> 2][4 * (k & 3) + 2], O[k >> 2][4 * (k & 3) + 3]));
-      st4_agent(mine, 64 * 64 * 4 + 16 * lane, make_float4(m, l, (float)E, 0.f));
+      st4_agent(mine, 64 * 64 * 4 + 16 * lane, make_float4(m, l, __builtin_bit_cast(float, g), 0.f));
       __builtin_amdgcn_s_waitcnt(0);  // this wave's state has been stored
       __syncthreads();
       unsigned *ctr = a.counters + ((long long)h * a.n_units + u) * kCounterStride;
@@ -674,23 +706,23 @@ void prefill_split_kernel(PrefillRunsArgs a) {
       if (!last) return;  // s_last is written again only past the next tile's barrier
       if (tid == 0) __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       struct State {
-        float4 o[16], mle;
+        float4 o[16], mlg;
       };
       auto load = [&](State &x, int c) {
         const __amdgpu_buffer_rsrc_t src = state(c);
 #pragma unroll
         for (int k = 0; k < 16; ++k) x.o[k] = ld4_agent(src, lane * 16, 1024 * k);
-        x.mle = ld4_agent(src, 64 * 64 * 4 + 16 * lane);
+        x.mlg = ld4_agent(src, 64 * 64 * 4 + 16 * lane);
       };
       auto add = [&](const State &x) {
-        const float mn = fmaxf(m, x.mle.x);
-        const int xe = (int)x.mle.z, en = min(E, xe);
-        float wa = fast_exp2(m - mn), wb = fast_exp2(x.mle.x - mn);
-        l = l * wa + x.mle.y * wb;
+        // whole-number exponents: every factor is a power of two, 1 at most
+        const float mn = fmaxf(m, x.mlg.x);
+        const int da = (int)fminf(mn - m, (float)kMaxShift), db = (int)fminf(mn - x.mlg.x, (float)kMaxShift);
+        const int ga = g + da, gb = __builtin_bit_cast(int, x.mlg.z) + db;
+        l = ldexpf(l, -da) + ldexpf(x.mlg.y, -db);
         m = mn;
-        wa = ldexpf(wa, en - E);
-        wb = ldexpf(wb, en - xe);
-        E = en;
+        g = min(ga, gb);
+        const float wa = ldexpf(1.0f, g - ga), wb = ldexpf(1.0f, g - gb);
 #pragma unroll
         for (int k = 0; k < 16; ++k) {
           floatx16 &o = O[k >> 2];
@@ -716,8 +748,8 @@ void prefill_split_kernel(PrefillRunsArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         st4(op + 32 * (r >> 2) + 4 * (r & 3),
-            make_float4(ldexpf(O[0][r] * inv, -(E + kPShift)), ldexpf(O[1][r] * inv, -(E + kPShift)),
-                        ldexpf(O[2][r] * inv, -(E + kPShift)), ldexpf(O[3][r] * inv, -(E + kPShift))));
+            make_float4(ldexpf(O[0][r] * inv, -g), ldexpf(O[1][r] * inv, -g),
+                        ldexpf(O[2][r] * inv, -g), ldexpf(O[3][r] * inv, -g)));
     }
     SP_STAMP(kPfStored);
   };
@@ -726,7 +758,7 @@ void prefill_split_kernel(PrefillRunsArgs a) {
   fetch(0);
   bool first = true;  // the run's first piece
   while (true) {
-    begin(__builtin_amdgcn_readfirstlane(word.y));
+    begin();
     SP_STAMP(kPfReady);
     do {
       __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's copies have landed

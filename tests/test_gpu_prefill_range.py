@@ -68,6 +68,18 @@ def worst(out, ref, by):
     return (d / r.clamp_min(1e-300)).max().item()
 
 
+def check(monkeypatch, q, kc, vc, start, by=("column", "row"), rows=None):
+    """The split launch is as close to 64 bits as the fp32 launch (half as much
+    again: other orders of the same sums) or within fp32's own rounding of a
+    product and a sum, 2^-21."""
+    ref = attend64(q, kc, vc, start)
+    outs = [attend(monkeypatch, split, q, kc, vc, start).reshape(ref.shape) for split in (0, 1)]
+    for b in by:
+        e0, e1 = (worst(o[rows] if rows else o, ref[rows] if rows else ref, b) for o in outs)
+        print(f"[error] by {b}: fp32 {e0:.2e} split {e1:.2e}", flush=True)
+        assert e1 <= max(1.5 * e0, 2.0 ** -21), (b, e0, e1)
+
+
 # a constant V: the output is that value, whatever is added up on the way
 @pytest.mark.parametrize("c", [1e30, 1e33, 1e36, 3e38])
 @pytest.mark.parametrize("marked", [False, True])
@@ -100,3 +112,37 @@ def test_exponent_rounding(monkeypatch):
     # a pair leaves out 2^-22 of a product at most; over 128 dims and 32 keys of
     # either sign it is a quarter of that at most
     assert e1 <= e0 + 2.0 ** -24, (e0, e1)
+
+
+# tiles that set no scale (zeros) or go through fp32 products (rows far apart)
+# before V of another magnitude, at the start of the line and inside it
+@pytest.mark.parametrize("scale", [1e-10, 1e-17, 1e-20, 1e-25, 1e-30])
+@pytest.mark.parametrize("kind", ["zero", "marked", "both"])
+def test_first_tiles(monkeypatch, scale, kind):
+    case(f"split prefill, {kind} tiles before V of {scale}")
+    n, start = 608, 96
+    q, kc, vc = normal(n, start, 13)
+    vc *= scale
+    for t in (0, 1, 5, 6, 11):
+        zero = kind == "zero" or (kind == "both" and t % 2 == 0)
+        if zero:
+            vc[:, 32 * t:32 * t + 32] = 0
+        else:
+            vc[:, 32 * t + 7] *= 2.0 ** -20
+    check(monkeypatch, q, kc, vc, start)
+
+
+# weights that fall and rise again by more than fp16 holds, from tile to tile
+@pytest.mark.parametrize("step", [8.0, 20.0])
+def test_weights_apart(monkeypatch, step):
+    case(f"split prefill, key tiles {step} apart")
+    import torch
+
+    n, start = 640, 64
+    q, kc, vc = normal(n, start, 15)
+    q *= 0.5
+    q[:, ::D] = 1.0
+    level = torch.arange(start + n, device="cuda") // 32 % 3  # 0, 1, 2, 0, ...
+    kc[:, :, 0] = level * step * D ** 0.5
+    vc *= torch.exp2(-level * step * 1.4427)[None, :, None]  # all tiles count
+    check(monkeypatch, q, kc, vc, start, by=("column", "row"))
