@@ -47,9 +47,20 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 #endif
 
 constexpr int kHalfTile = kSplitTileFloats / 2;  // floats of a tile's K (or V) part
+// The low half of a V pair is stored times 2^12, where it is as large as the
+// high half at most.  Then fp16's subnormals cut off at 2^-37 of a scaled value:
+// down to 2^-28 of the tile's largest h + l holds a value to 2^-23 of it.
+constexpr int kLowScale = 4096;
+constexpr int kElemRange = 28;
+// V rows: a weight's pair cuts off at 2^-36 of the tile's largest (typically;
+// 2^-26 at worst), so a row of 2^-12 of the tile's largest value or less -- a
+// zero row too -- under the largest weight could leave an output to weights
+// that have lost bits.
+constexpr int kVRowRange = 12;
 
-// x0 .. x7 (already scaled) -> h and l: two conversions of a pair (v_cvt_pk)
-// and one subtraction that reads h as it is (v_fma_mix) per value.
+// x0 .. x7 (already scaled) -> h and l times LOW: two conversions of a pair
+// (v_cvt_pk) and one subtraction that reads h as it is (v_fma_mix) per value.
+template <int LOW>
 __device__ __forceinline__ void split8(const float (&x)[8], half8 &h, half8 &l) {
   typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
   typedef float float2_t __attribute__((ext_vector_type(2)));
@@ -61,6 +72,7 @@ __device__ __forceinline__ void split8(const float (&x)[8], half8 &h, half8 &l) 
     const unsigned ab = __builtin_bit_cast(unsigned, a);
     asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r.x) : "v"(ab), "v"(x[i]));
     asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r.y) : "v"(ab), "v"(x[i + 1]));
+    if (LOW != 1) r *= (float)LOW;
     const half2_t b = __builtin_convertvector(r, half2_t);
     h[i] = a.x;
     h[i + 1] = a.y;
@@ -127,17 +139,19 @@ __device__ __forceinline__ unsigned wave_red(unsigned v) {
 
 // Tile word: scale exponent + 128 in bits 0..7, kSplitFp32 and kSplitZero.
 constexpr int kSplitFp32 = 0x100, kSplitZero = 0x200;
-// From the largest and the smallest nonzero row maximum (bits; ~0: no
-// nonzero row): fp32 for infinities and NaN, for rows whose largest value is
-// below 2^-15 of the tile's (an fp16 subnormal would cut them off above
-// 2^-24 of that value) and for tiles whose scale would pass 2^126.  A marked
-// tile's exponent says how large its values are: O takes it for its own.
-__device__ __forceinline__ int tile_word(unsigned mx, unsigned mn) {
-  constexpr unsigned kSplitRange = 15;
+// From the tile's largest magnitude (bits), its smallest row maximum and one
+// less than its smallest nonzero magnitude (~0: none): fp32 products for
+// infinities and NaN, for tiles whose scale would pass 2^126, for rows whose
+// largest value is below 2^-row_range of the tile's and for values below
+// 2^-elem_range of it.  A marked tile's exponent says how large its values are:
+// O takes it for its own.
+__device__ __forceinline__ int tile_word(unsigned mx, unsigned row_min, int row_range, unsigned elem_min,
+                                         int elem_range) {
   if (mx == 0) return 128 | kSplitZero;
-  const unsigned e = mx >> 23;
-  const int word = scale_exp(mx) + 128;
-  return e == 255 || e < 15 || (mn >> 23) + kSplitRange < e ? word | kSplitFp32 : word;
+  const int e = (int)(mx >> 23), word = scale_exp(mx) + 128;
+  const bool fp32 = e == 255 || e < 15 || (int)(row_min >> 23) + row_range < e ||
+                    (int)(elem_min >> 23) < max(1, e - elem_range);
+  return fp32 ? word | kSplitFp32 : word;
 }
 // The scale exponent that a V tile asks of O.  A marked tile's values are not
 // scaled: the limits keep its weights, 2^(15 + exponent) at most, and their
@@ -197,7 +211,7 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
     }
     return;
   }
-  __shared__ unsigned s_row[2][32], s_vmax[2], s_vmin[2];
+  __shared__ unsigned s_row[2][32], s_vmax[2], s_vmin[2], s_velem[2];
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int hl = lane >> 5, col = lane & 31;
   const int h = (int)blockIdx.x % a.n_kv, kt = (int)blockIdx.x / a.n_kv;
@@ -216,19 +230,23 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
                                : a.v_cache + h * a.kv_stride + (long long)row * kHeadDim;
       x[i] = row < rows ? ld4(src + 4 * col) : zero;
     }
-    unsigned mx = 0, mn = ~0u;
+    unsigned mx = 0, mn = ~0u, en = ~0u;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const unsigned r = half_red<true>(
-          max(max(abs_bits(x[i].x), abs_bits(x[i].y)), max(abs_bits(x[i].z), abs_bits(x[i].w))));
+      const int row = 32 * kt + 16 * t + 8 * (i >> 2) + 4 * hl + (i & 3);
+      const unsigned b[4] = {abs_bits(x[i].x), abs_bits(x[i].y), abs_bits(x[i].z), abs_bits(x[i].w)};
+      en = min(en, min(min(b[0] - 1, b[1] - 1), min(b[2] - 1, b[3] - 1)));  // zeros wrap to ~0
+      const unsigned r = half_red<true>(max(max(b[0], b[1]), max(b[2], b[3])));
       mx = max(mx, r);
-      mn = min(mn, r ? r : ~0u);
+      mn = min(mn, row < rows ? r : ~0u);
     }
     mx = wave_red<true>(mx);
     mn = wave_red<false>(mn);
+    en = wave_red<false>(en);
     if (lane == 0) {
       s_vmax[t] = mx;
       s_vmin[t] = mn;
+      s_velem[t] = en;
     }
     if (ROPE) {
 #pragma unroll
@@ -239,7 +257,8 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
       }
     }
     __syncthreads();
-    const int word = tile_word(max(s_vmax[0], s_vmax[1]), min(s_vmin[0], s_vmin[1]));
+    const int word = tile_word(max(s_vmax[0], s_vmax[1]), min(s_vmin[0], s_vmin[1]), kVRowRange,
+                               min(s_velem[0], s_velem[1]), kElemRange);
     const bool marked = (word & kSplitFp32) != 0;
     const float sc = exp2i((word & 255) - 128);
     float *dst = tile + kHalfTile + t * 8 * 256 + 4 * lane;
@@ -250,7 +269,7 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
       for (int i = 0; i < 8; ++i)
         y[i] = marked ? 0.f : (db == 0 ? x[i].x : db == 1 ? x[i].y : db == 2 ? x[i].z : x[i].w) * sc;
       half8 hv, lv;
-      split8(y, hv, lv);
+      split8<kLowScale>(y, hv, lv);
       *reinterpret_cast<half8 *>(dst + 512 * db) = hv;
       *reinterpret_cast<half8 *>(dst + 512 * db + 256) = lv;
     }
@@ -312,7 +331,7 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
   if (hl == 0) s_row[w][col] = mx;
   __syncthreads();
   mx = max(s_row[0][col], s_row[1][col]);
-  const int word = tile_word(wave_red<true>(mx), wave_red<false>(mx ? mx : ~0u));
+  const int word = tile_word(wave_red<true>(mx), wave_red<false>(mx ? mx : ~0u), 15, ~0u, 0);
   const bool marked = (word & kSplitFp32) != 0;
   const float sc = exp2i((word & 255) - 128);
 #pragma unroll
@@ -324,7 +343,7 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
       const float y[8] = {e0.x * sc, e0.y * sc, e0.z * sc, e0.w * sc,
                           e1.x * sc, e1.y * sc, e1.z * sc, e1.w * sc};
       half8 hv, lv;
-      split8(y, hv, lv);
+      split8<1>(y, hv, lv);
       float *dst = tile + (2 * w + u + 4 * half) * 512 + 4 * lane;
       *reinterpret_cast<half8 *>(dst) = hv;
       *reinterpret_cast<half8 *>(dst + 256) = lv;
@@ -525,9 +544,10 @@ void prefill_split_kernel(PrefillRunsArgs a) {
       mm(x[2 * i], qh[s + i], S);
     }
   };
-  auto mm_o = [&](const half8 (&x)[4], int db, half8 ph, half8 pl) {  // dim blocks db, db + 1
-    mm(x[1], ph, O[db]);
-    mm(x[3], ph, O[db + 1]);
+  // Dim blocks db, db + 1; pq: ph over the scale of V's low half.
+  auto mm_o = [&](const half8 (&x)[4], int db, half8 ph, half8 pl, half8 pq) {
+    mm(x[1], pq, O[db]);
+    mm(x[3], pq, O[db + 1]);
     mm(x[0], pl, O[db]);
     mm(x[2], pl, O[db + 1]);
     mm(x[0], ph, O[db]);
@@ -612,16 +632,19 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     // fp32 products come after these, whose factor is then 0 (a branch around
     // them would cost 24 more registers than there are)
     const float f = fp32_v ? 0.f : ldexpf(1.0f, min(g - ev, kMaxFactor));
-    half8 ph, pl;
+    const _Float16 down = (_Float16)(1.0f / kLowScale);
+    half8 ph, pl, pq;
     split8f(p, 0, f, ph, pl);
+    pq = ph * down;
     rd(B, dv, 4);
-    mm_o(A, 0, ph, pl);
+    mm_o(A, 0, ph, pl, pq);
     rd(A, dv, 8);
-    mm_o(B, 2, ph, pl);
+    mm_o(B, 2, ph, pl, pq);
     rd(B, dv, 12);
     split8f(p, 8, f, ph, pl);
-    mm_o(A, 0, ph, pl);
-    mm_o(B, 2, ph, pl);
+    pq = ph * down;
+    mm_o(A, 0, ph, pl, pq);
+    mm_o(B, 2, ph, pl, pq);
     if (fp32_v) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) p[r] = ldexpf(p[r], g);
@@ -657,7 +680,7 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     for (int s = 0; s < 8; ++s) {
       const float4 v = x[2 * s], w = x[2 * s + 1];
       const float y[8] = {v.x * sc, v.y * sc, v.z * sc, v.w * sc, w.x * sc, w.y * sc, w.z * sc, w.w * sc};
-      split8(y, qh[s], ql[s]);
+      split8<1>(y, qh[s], ql[s]);
     }
 #pragma unroll
     for (int db = 0; db < 4; ++db) O[db] = floatx16{};

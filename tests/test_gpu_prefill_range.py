@@ -4,6 +4,7 @@ between tiles -- against 64 bits, each output column and each query row by
 itself, beside the fp32 launches on the same inputs."""
 import sys
 
+import numpy as np
 import pytest
 
 from common import D
@@ -132,6 +133,23 @@ def test_first_tiles(monkeypatch, scale, kind):
     check(monkeypatch, q, kc, vc, start)
 
 
+# a sink: its key takes nearly all of the weight and its value is small or zero
+@pytest.mark.parametrize("gap,v", [(12.0, 0.0), (25.0, 0.0), (40.0, 0.0), (6.0, 2.0 ** -9), (9.0, 2.0 ** -13),
+                                   (14.0, 2.0 ** -20)])
+@pytest.mark.parametrize("rows", [1, 32])
+def test_sink(monkeypatch, gap, v, rows):
+    case(f"split prefill, {rows} sink rows {gap} above the rest, values {v}")
+    n, start = 640, 0
+    q, kc, vc = normal(n, start, 14)
+    q *= 0.5
+    q[:, ::D] = 1.0
+    kc[:, :, 0] = 0.0
+    kc[:, :rows] = 0.0
+    kc[:, :rows, 0] = gap * D ** 0.5
+    vc[:, :rows] *= v
+    check(monkeypatch, q, kc, vc, start, by=("row",), rows=slice(33, None))
+
+
 # weights that fall and rise again by more than fp16 holds, from tile to tile
 @pytest.mark.parametrize("step", [8.0, 20.0])
 def test_weights_apart(monkeypatch, step):
@@ -146,3 +164,25 @@ def test_weights_apart(monkeypatch, step):
     kc[:, :, 0] = level * step * D ** 0.5
     vc *= torch.exp2(-level * step * 1.4427)[None, :, None]  # all tiles count
     check(monkeypatch, q, kc, vc, start, by=("column", "row"))
+
+
+RATIOS = [2.0 ** 14, 2.0 ** 20, 2.0 ** 25, 2.0 ** 30, 2.0 ** 40, 2.0 ** 60]
+
+
+# V: one head dim far above the rest, some rows, dims spread evenly; by column
+# where one dim makes up a row's norm (its sum may be near zero)
+@pytest.mark.parametrize("r", RATIOS)
+@pytest.mark.parametrize("kind", ["dim", "rows", "spread"])
+def test_v_apart(monkeypatch, kind, r):
+    case(f"split prefill, V {kind} {r} apart")
+    import torch
+
+    n, start = 544, 64
+    q, kc, vc = normal(n, start, 16)
+    if kind == "dim":
+        vc[:, :, 5] *= r
+    elif kind == "rows":
+        vc[:, ::7] *= r
+    else:
+        vc *= torch.exp2(torch.linspace(0, 1, D, device="cuda") * float(np.log2(r)))
+    check(monkeypatch, q, kc, vc, start, by=("column",) if kind == "dim" else ("column", "row"))
