@@ -47,9 +47,9 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 #endif
 
 constexpr int kHalfTile = kSplitTileFloats / 2;  // floats of a tile's K (or V) part
-// The low half of a V pair is stored times 2^12, where it is as large as the
-// high half at most.  Then fp16's subnormals cut off at 2^-37 of a scaled value:
-// down to 2^-28 of the tile's largest h + l holds a value to 2^-23 of it.
+// The low half of a pair is stored times 2^12, where it is as large as the high
+// half at most.  Then fp16's subnormals cut off at 2^-37 of a scaled value: down
+// to 2^-28 of the largest h + l holds a value to 2^-23 of it.
 constexpr int kLowScale = 4096;
 constexpr int kElemRange = 28;
 // V rows: a weight's pair cuts off at 2^-36 of the tile's largest (typically;
@@ -103,6 +103,13 @@ __device__ __forceinline__ void split8f(const float (&p)[16], int r, float f, ha
 __device__ __forceinline__ unsigned abs_bits(float x) {
   return __builtin_bit_cast(unsigned, x) & 0x7fffffffu;
 }
+// The largest magnitude and one less than the smallest nonzero one (zeros wrap
+// to ~0) of x and what came before.
+__device__ __forceinline__ void mag4(float4 x, unsigned &mx, unsigned &elem_min) {
+  const unsigned b[4] = {abs_bits(x.x), abs_bits(x.y), abs_bits(x.z), abs_bits(x.w)};
+  mx = max(mx, max(max(b[0], b[1]), max(b[2], b[3])));
+  elem_min = min(elem_min, min(min(b[0] - 1, b[1] - 1), min(b[2] - 1, b[3] - 1)));
+}
 __device__ __forceinline__ float exp2i(int e) {  // 2^e, -126 <= e <= 127
   return __builtin_bit_cast(float, (unsigned)(e + 127) << 23);
 }
@@ -139,19 +146,28 @@ __device__ __forceinline__ unsigned wave_red(unsigned v) {
 
 // Tile word: scale exponent + 128 in bits 0..7, kSplitFp32 and kSplitZero.
 constexpr int kSplitFp32 = 0x100, kSplitZero = 0x200;
-// From the tile's largest magnitude (bits), its smallest row maximum and one
-// less than its smallest nonzero magnitude (~0: none): fp32 products for
-// infinities and NaN, for tiles whose scale would pass 2^126, for rows whose
-// largest value is below 2^-row_range of the tile's and for values below
-// 2^-elem_range of it.  A marked tile's exponent says how large its values are:
-// O takes it for its own.
-__device__ __forceinline__ int tile_word(unsigned mx, unsigned row_min, int row_range, unsigned elem_min,
-                                         int elem_range) {
+// Whether values whose largest magnitude has these bits, and whose smallest
+// nonzero one has elem_min + 1 (~0: none), do not fit pairs: an infinity or a
+// NaN, a scale past 2^126, a value below 2^-28 of the largest.
+__device__ __forceinline__ bool no_pairs(unsigned mx, unsigned elem_min) {
+  const int e = (int)(mx >> 23);
+  return e == 255 || e < 15 || (int)(elem_min >> 23) < max(1, e - kElemRange);
+}
+// A V tile's word; row_min is its smallest row maximum.  A marked tile's
+// exponent says how large its values are: O takes it for its own.
+__device__ __forceinline__ int v_word(unsigned mx, unsigned row_min, unsigned elem_min) {
   if (mx == 0) return 128 | kSplitZero;
-  const int e = (int)(mx >> 23), word = scale_exp(mx) + 128;
-  const bool fp32 = e == 255 || e < 15 || (int)(row_min >> 23) + row_range < e ||
-                    (int)(elem_min >> 23) < max(1, e - elem_range);
-  return fp32 ? word | kSplitFp32 : word;
+  const bool fp32 = no_pairs(mx, elem_min) || (int)(row_min >> 23) + kVRowRange < (int)(mx >> 23);
+  return (scale_exp(mx) + 128) | (fp32 ? kSplitFp32 : 0);
+}
+// A K tile's.  Values past 2^54 are marked: the scales of K and q and their
+// product then stay inside fp32 (a score may be small all the same, where K
+// or q has zeros).
+constexpr int kQkTop = 127 + 54;
+__device__ __forceinline__ int k_word(unsigned mx, unsigned elem_min) {
+  if (mx == 0) return 128 | kSplitZero;
+  const bool fp32 = no_pairs(mx, elem_min) || (int)(mx >> 23) > kQkTop;
+  return (scale_exp(mx) + 128) | (fp32 ? kSplitFp32 : 0);
 }
 // The scale exponent that a V tile asks of O.  A marked tile's values are not
 // scaled: the limits keep its weights, 2^(15 + exponent) at most, and their
@@ -211,7 +227,7 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
     }
     return;
   }
-  __shared__ unsigned s_row[2][32], s_vmax[2], s_vmin[2], s_velem[2];
+  __shared__ unsigned s_vmax[2], s_vmin[2], s_velem[2], s_kmax[2], s_kelem[2];
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int hl = lane >> 5, col = lane & 31;
   const int h = (int)blockIdx.x % a.n_kv, kt = (int)blockIdx.x / a.n_kv;
@@ -234,9 +250,9 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int row = 32 * kt + 16 * t + 8 * (i >> 2) + 4 * hl + (i & 3);
-      const unsigned b[4] = {abs_bits(x[i].x), abs_bits(x[i].y), abs_bits(x[i].z), abs_bits(x[i].w)};
-      en = min(en, min(min(b[0] - 1, b[1] - 1), min(b[2] - 1, b[3] - 1)));  // zeros wrap to ~0
-      const unsigned r = half_red<true>(max(max(b[0], b[1]), max(b[2], b[3])));
+      unsigned r = 0;
+      mag4(x[i], r, en);
+      r = half_red<true>(r);
       mx = max(mx, r);
       mn = min(mn, row < rows ? r : ~0u);
     }
@@ -257,8 +273,7 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
       }
     }
     __syncthreads();
-    const int word = tile_word(max(s_vmax[0], s_vmax[1]), min(s_vmin[0], s_vmin[1]), kVRowRange,
-                               min(s_velem[0], s_velem[1]), kElemRange);
+    const int word = v_word(max(s_vmax[0], s_vmax[1]), min(s_vmin[0], s_vmin[1]), min(s_velem[0], s_velem[1]));
     const bool marked = (word & kSplitFp32) != 0;
     const float sc = exp2i((word & 255) - 128);
     float *dst = tile + kHalfTile + t * 8 * 256 + 4 * lane;
@@ -315,23 +330,22 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
       }
     }
   }
-  unsigned mx = 0;
+  unsigned mx = 0, en = ~0u;
 #pragma unroll
   for (int u = 0; u < 2; ++u)
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
-      const float4 l4 = lo[u][e], h4 = hi[u][e];
-      mx = max(mx, max(max(abs_bits(l4.x), abs_bits(l4.y)), max(abs_bits(l4.z), abs_bits(l4.w))));
-      mx = max(mx, max(max(abs_bits(h4.x), abs_bits(h4.y)), max(abs_bits(h4.z), abs_bits(h4.w))));
+      mag4(lo[u][e], mx, en);
+      mag4(hi[u][e], mx, en);
     }
-  {
-    const auto r = __builtin_amdgcn_permlane32_swap(mx, mx, false, false);
-    mx = max((unsigned)r[0], (unsigned)r[1]);
+  mx = wave_red<true>(mx);
+  en = wave_red<false>(en);
+  if (lane == 0) {
+    s_kmax[w] = mx;
+    s_kelem[w] = en;
   }
-  if (hl == 0) s_row[w][col] = mx;
   __syncthreads();
-  mx = max(s_row[0][col], s_row[1][col]);
-  const int word = tile_word(wave_red<true>(mx), wave_red<false>(mx ? mx : ~0u), 15, ~0u, 0);
+  const int word = k_word(max(s_kmax[0], s_kmax[1]), min(s_kelem[0], s_kelem[1]));
   const bool marked = (word & kSplitFp32) != 0;
   const float sc = exp2i((word & 255) - 128);
 #pragma unroll
@@ -343,7 +357,7 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
       const float y[8] = {e0.x * sc, e0.y * sc, e0.z * sc, e0.w * sc,
                           e1.x * sc, e1.y * sc, e1.z * sc, e1.w * sc};
       half8 hv, lv;
-      split8<1>(y, hv, lv);
+      split8<kLowScale>(y, hv, lv);
       float *dst = tile + (2 * w + u + 4 * half) * 512 + 4 * lane;
       *reinterpret_cast<half8 *>(dst) = hv;
       *reinterpret_cast<half8 *>(dst + 256) = lv;
@@ -536,10 +550,11 @@ void prefill_split_kernel(PrefillRunsArgs a) {
   auto mm = [](half8 x, half8 y, floatx16 &acc) {
     acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(x, y, acc, 0, 0, 0);
   };
-  auto mm_s = [&](floatx16 &S, const half8 (&x)[4], int s) {  // steps s, s + 1
+  // Steps s, s + 1; L: products with K's low half, times its scale.
+  auto mm_s = [&](floatx16 &S, floatx16 &L, const half8 (&x)[4], int s) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      mm(x[2 * i + 1], qh[s + i], S);
+      mm(x[2 * i + 1], qh[s + i], L);
       mm(x[2 * i], ql[s + i], S);
       mm(x[2 * i], qh[s + i], S);
     }
@@ -557,17 +572,19 @@ void prefill_split_kernel(PrefillRunsArgs a) {
   // The products of one tile (operands at dk, words wk and wv).
   auto step = [&](const float *dk, int kt, int wk, int wv) {
     const float *dv = dk + kHalfTile;
-    floatx16 S = floatx16{};
+    floatx16 S = floatx16{}, L = floatx16{};
     half8 A[4], B[4];
     rd(A, dk, 0);
     rd(B, dk, 4);
-    mm_s(S, A, 0);
+    mm_s(S, L, A, 0);
     rd(A, dk, 8);
-    mm_s(S, B, 2);
+    mm_s(S, L, B, 2);
     rd(B, dk, 12);
-    mm_s(S, A, 4);
+    mm_s(S, L, A, 4);
     rd(A, dv, 0);
-    mm_s(S, B, 6);
+    mm_s(S, L, B, 6);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) S[r] = fmaf(L[r], 1.0f / kLowScale, S[r]);
     float c = fmaxf(cq * exp2i(128 - (wk & 255)), 1e-37f);  // > 0: a masked -inf stays -inf
     // A marked part's operands are zeros; its products come from the cache.
     if (wk & kSplitFp32) {

@@ -186,3 +186,15 @@ def test_v_apart(monkeypatch, kind, r):
     else:
         vc *= torch.exp2(torch.linspace(0, 1, D, device="cuda") * float(np.log2(r)))
     check(monkeypatch, q, kc, vc, start, by=("column",) if kind == "dim" else ("column", "row"))
+
+
+# K: one head dim far above the rest, q zero or as far below the rest there
+@pytest.mark.parametrize("r", RATIOS)
+@pytest.mark.parametrize("other", ["zero", "inverse"])
+def test_k_apart(monkeypatch, other, r):
+    case(f"split prefill, a K dim of {r}, q {other}")
+    n, start = 544, 64
+    q, kc, vc = normal(n, start, 16)
+    kc[:, :, 5] *= r
+    q.view(n, HQ, D)[:, :, 5] *= 0.0 if other == "zero" else 1 / r
+    check(monkeypatch, q, kc, vc, start)
