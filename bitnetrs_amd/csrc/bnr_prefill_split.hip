@@ -537,6 +537,7 @@ void prefill_split_kernel(PrefillRunsArgs a) {
   floatx16 O[4];
   float cq, m, l;
   int g, g_cap, qrow, q0;
+  bool fp32_q;  // a query of the wave's does not fit pairs (uniform)
   const float *qp;
 
   // Four operands read ahead of the products that use them (two sets of
@@ -550,12 +551,12 @@ void prefill_split_kernel(PrefillRunsArgs a) {
   auto mm = [](half8 x, half8 y, floatx16 &acc) {
     acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(x, y, acc, 0, 0, 0);
   };
-  // Steps s, s + 1; L: products with K's low half, times its scale.
+  // Steps s, s + 1; L: products with a low half, times its scale.
   auto mm_s = [&](floatx16 &S, floatx16 &L, const half8 (&x)[4], int s) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       mm(x[2 * i + 1], qh[s + i], L);
-      mm(x[2 * i], ql[s + i], S);
+      mm(x[2 * i], ql[s + i], L);
       mm(x[2 * i], qh[s + i], S);
     }
   };
@@ -587,7 +588,7 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     for (int r = 0; r < 16; ++r) S[r] = fmaf(L[r], 1.0f / kLowScale, S[r]);
     float c = fmaxf(cq * exp2i(128 - (wk & 255)), 1e-37f);  // > 0: a masked -inf stays -inf
     // A marked part's operands are zeros; its products come from the cache.
-    if (wk & kSplitFp32) {
+    if ((wk & kSplitFp32) || fp32_q) {
       S = sp_fp32_s(a, h, kt, qp);
       c = a.scale_log2;
     }
@@ -670,7 +671,8 @@ void prefill_split_kernel(PrefillRunsArgs a) {
   };
 
   // Queries of the unit's block: lane's dims 16 s + 8 hl + i of query q0 + col
-  // (rows past the end repeat the last and are not stored), as fp16 pairs.
+  // (rows past the end repeat the last and are not stored), as fp16 pairs.  A
+  // query that does not fit them takes its wave through fp32 scores.
   auto begin = [&] {
     int lane = tid & 63;
     asm volatile("" : "+v"(lane));
@@ -679,17 +681,19 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     qrow = min(q0 + col, a.n_tokens - 1);
     qp = a.q + ((long long)qrow * a.n_heads + head) * kHeadDim;
     float4 x[16];
-    unsigned mx = 0;
+    unsigned mx = 0, en = ~0u;
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       x[2 * s] = ld4(qp + 16 * s + 8 * hl);
       x[2 * s + 1] = ld4(qp + 16 * s + 8 * hl + 4);
     }
 #pragma unroll
-    for (int s = 0; s < 16; ++s)
-      mx = max(mx, max(max(abs_bits(x[s].x), abs_bits(x[s].y)), max(abs_bits(x[s].z), abs_bits(x[s].w))));
+    for (int s = 0; s < 16; ++s) mag4(x[s], mx, en);
     const auto r = __builtin_amdgcn_permlane32_swap(mx, mx, false, false);
     mx = max((unsigned)r[0], (unsigned)r[1]);
+    const auto re = __builtin_amdgcn_permlane32_swap(en, en, false, false);
+    en = min((unsigned)re[0], (unsigned)re[1]);
+    fp32_q = __ballot(mx != 0 && (no_pairs(mx, en) || (int)(mx >> 23) > kQkTop)) != 0;
     const int e = scale_exp(mx);
     const float sc = exp2i(e);
     cq = ldexpf(a.scale_log2, -e);
@@ -697,7 +701,7 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     for (int s = 0; s < 8; ++s) {
       const float4 v = x[2 * s], w = x[2 * s + 1];
       const float y[8] = {v.x * sc, v.y * sc, v.z * sc, v.w * sc, w.x * sc, w.y * sc, w.z * sc, w.w * sc};
-      split8<1>(y, qh[s], ql[s]);
+      split8<kLowScale>(y, qh[s], ql[s]);
     }
 #pragma unroll
     for (int db = 0; db < 4; ++db) O[db] = floatx16{};

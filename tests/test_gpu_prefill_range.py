@@ -198,3 +198,62 @@ def test_k_apart(monkeypatch, other, r):
     kc[:, :, 5] *= r
     q.view(n, HQ, D)[:, :, 5] *= 0.0 if other == "zero" else 1 / r
     check(monkeypatch, q, kc, vc, start)
+
+
+# q: one head dim far above the rest, K zero or as far below the rest there; in
+# every row or in a few
+@pytest.mark.parametrize("r", RATIOS)
+@pytest.mark.parametrize("other", ["zero", "inverse"])
+@pytest.mark.parametrize("every", [1, 50])
+def test_q_apart(monkeypatch, other, every, r):
+    case(f"split prefill, a q dim of {r} in every {every} rows, K {other}")
+    n, start = 544, 64
+    q, kc, vc = normal(n, start, 16)
+    q.view(n, HQ, D)[::every, :, 5] *= r
+    kc[:, :, 5] *= 0.0 if other == "zero" else 1 / r
+    check(monkeypatch, q, kc, vc, start)
+
+
+# q and K spread evenly over the dims, against one another
+@pytest.mark.parametrize("r", RATIOS)
+def test_q_and_k_spread(monkeypatch, r):
+    case(f"split prefill, q and K spread over {r}")
+    import torch
+
+    n, start = 544, 64
+    q, kc, vc = normal(n, start, 16)
+    spread = torch.exp2(torch.linspace(0, 1, D, device="cuda") * float(np.log2(r)))
+    q.view(n, HQ, D).mul_(spread)
+    check(monkeypatch, q, kc / spread, vc, start)
+
+
+# magnitudes at the ends of fp32: products of q and K stay in range
+@pytest.mark.parametrize("qs,ks", [(2.0 ** 90, 2.0 ** -90), (2.0 ** -90, 2.0 ** 90), (2.0 ** -110, 2.0 ** 110),
+                                   (2.0 ** 110, 2.0 ** -110), (2.0 ** -60, 2.0 ** -60)])
+def test_magnitudes(monkeypatch, qs, ks):
+    case(f"split prefill, q of {qs}, K of {ks}")
+    n, start = 544, 64
+    q, kc, vc = normal(n, start, 17)
+    check(monkeypatch, q * qs, kc * ks, vc, start)
+
+
+def test_large_q_and_k_apart(monkeypatch):
+    """q and K near 2^100 in head dims where the other is zero: their scales'
+    product leaves fp32 although every score is small."""
+    case("split prefill, q and K of 2^100 apart")
+    n, start = 544, 64
+    q, kc, vc = normal(n, start, 18)
+    qd = q.view(n, HQ, D)
+    qd[:, :, 3] = 2.0 ** 100
+    kc[:, :, 3] = 0
+    kc[:, :, 4] *= 2.0 ** 100
+    qd[:, :, 4] = 0
+    check(monkeypatch, q, kc, vc, start)
+
+
+# every head count per kv head the split kernels are built for
+@pytest.mark.parametrize("n_heads,n_kv", [(4, 2), (16, 2), (20, 5)])
+def test_heads(monkeypatch, n_heads, n_kv):
+    case(f"split prefill error at {n_heads}/{n_kv} heads")
+    q, kc, vc = normal(700, 45, 19, n_heads, n_kv)
+    check(monkeypatch, q, kc, vc, 45)
