@@ -31,6 +31,7 @@ namespace bnr {
 namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 // Timeline stamps of a measurement build (BNR_TIMELINE; PfStamp): wave 0's
@@ -187,6 +188,8 @@ __device__ __forceinline__ int v_exp(int word) {
 //   V, step t (16 keys), dim block db, part p: at 16 + 8 t + 2 db + p; lane l
 //     holds dim 4 (l % 32) + db of keys 16 t + 4 (l / 32) + {0..3} and 8 more:
 //     the keys that lane's registers 8 t .. 8 t + 7 of S^T hold.
+// A marked K part holds the fp32 values: dims + 0 .. 3 in place of h, + 4 .. 7 in
+// place of l.  A marked V part holds zeros.
 // Waves 0, 1 take V (step t = wave), waves 2, 3 take K (steps 2w', 2w'+1 and
 // the four dims blocks 64 further, so that a rotation pair sits in one lane).
 // Rows past the last cached one are zero.
@@ -348,21 +351,25 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
   const int word = k_word(max(s_kmax[0], s_kmax[1]), min(s_kelem[0], s_kelem[1]));
   const bool marked = (word & kSplitFp32) != 0;
   const float sc = exp2i((word & 255) - 128);
+  if (tid == 128) info->x = word;
 #pragma unroll
   for (int u = 0; u < 2; ++u)
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
-      const float4 e0 = marked ? zero : half ? hi[u][0] : lo[u][0];
-      const float4 e1 = marked ? zero : half ? hi[u][1] : lo[u][1];
+      const float4 e0 = half ? hi[u][0] : lo[u][0], e1 = half ? hi[u][1] : lo[u][1];
+      float *dst = tile + (2 * w + u + 4 * half) * 512 + 4 * lane;
+      if (marked) {
+        st4(dst, e0);
+        st4(dst + 256, e1);
+        continue;
+      }
       const float y[8] = {e0.x * sc, e0.y * sc, e0.z * sc, e0.w * sc,
                           e1.x * sc, e1.y * sc, e1.z * sc, e1.w * sc};
       half8 hv, lv;
       split8<kLowScale>(y, hv, lv);
-      float *dst = tile + (2 * w + u + 4 * half) * 512 + 4 * lane;
       *reinterpret_cast<half8 *>(dst) = hv;
       *reinterpret_cast<half8 *>(dst + 256) = lv;
     }
-  if (tid == 128) info->x = word;
 }
 
 // ---------------------------------------------------------------------------
@@ -411,40 +418,61 @@ constexpr int kNoScale = 1 << 28;   // O holds nothing yet
 constexpr int kMaxFactor = 112;     // of 2^(g - ev), a float
 constexpr int kMaxShift = 4096;     // more than any O keeps
 
-__device__ __forceinline__ float max_half_swap(float v) {  // max over lanes l, l ^ 32
+// Maximum and sum over lanes l, l ^ 32.
+__device__ __forceinline__ float max_half_swap(float v) {
   const unsigned u = __builtin_bit_cast(unsigned, v);
   const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
   return fmaxf(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
+}
+
+__device__ __forceinline__ float sum_half_swap(float v) {
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
 }
 
 __device__ __forceinline__ half8 ld_op(const float *lds, int op) {
   return *reinterpret_cast<const half8 *>(lds + op * 256 + 4 * (threadIdx.x & 63));
 }
 
-// S^T of a marked tile with fp32 products (v_mfma_f32_32x32x2_f32), K and q
-// read from memory: step kk takes dim 64 (lane / 32) + kk.  The caller's scale
-// is log2(e) / sqrt(d) alone.  Rows past the last repeat it (masked).
-__device__ __forceinline__ floatx16 sp_fp32_s(const PrefillRunsArgs &a, int h, int kt, const float *qp) {
-  const int lane = threadIdx.x & 63, hl = lane >> 5, col = lane & 31;
-  const int row = min(kt * 32 + col, a.start_pos + a.n_tokens - 1);
-  const float *kp = a.k_cache + h * a.kv_stride + (long long)row * kHeadDim + 64 * hl;
+// Value i of a pair operand, or of the fp32 values that take its place (x, y:
+// the two 16-byte words of the lane).
+__device__ __forceinline__ float op_value(half8 x, half8 y, int i, bool fp32, float unscale) {
+  const float pair = fmaf((float)y[i], 1.0f / kLowScale, (float)x[i]) * unscale;
+  const floatx4 v = __builtin_bit_cast(floatx4, i < 4 ? x : y);
+  return fp32 ? v[i & 3] : pair;
+}
+
+// S^T of a tile with fp32 products (v_mfma_f32_32x32x2_f32): step 8 s + i takes
+// dim 16 s + 8 (lane / 32) + i.  K and q each as pairs (unscale_k, unscale_q
+// undo their scales) or fp32 values.  The caller's scale is log2(e) / sqrt(d)
+// alone.
+__device__ __forceinline__ floatx16 sp_fp32_s(const float *dk, bool fp32_k, float unscale_k, const half8 (&qh)[8],
+                                              const half8 (&ql)[8], bool fp32_q, float unscale_q) {
   floatx16 S = floatx16{};
-#pragma unroll 1
-  for (int i = 0; i < 16; ++i) {
-    const float4 kv = ld4(kp + 4 * i), qv = ld4(qp + 64 * hl + 4 * i);
-    S = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.x, qv.x, S, 0, 0, 0);
-    S = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.y, qv.y, S, 0, 0, 0);
-    S = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.z, qv.z, S, 0, 0, 0);
-    S = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.w, qv.w, S, 0, 0, 0);
+  // hidden from the compiler, which would otherwise form q's 64 values ahead of
+  // the tile loop and keep them in registers
+  asm volatile("" : "+v"(unscale_q));
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    __builtin_amdgcn_sched_barrier(0);
+    const half8 x = ld_op(dk, 2 * s), y = ld_op(dk, 2 * s + 1);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      S = __builtin_amdgcn_mfma_f32_32x32x2f32(op_value(x, y, i, fp32_k, unscale_k),
+                                               op_value(qh[s], ql[s], i, fp32_q, unscale_q), S, 0, 0, 0);
   }
+  __builtin_amdgcn_sched_barrier(0);
   return S;
 }
 
-// O^T += V^T P^T of a marked tile with fp32 products: step s takes key
-// 8 (s / 4) + 4 (lane / 32) + s % 4.
+// O^T += V^T P^T with fp32 products, V read from the cache: step s takes key
+// 8 (s / 4) + 4 (lane / 32) + s % 4.  Rows past the last repeat it (masked).
 __device__ __forceinline__ void sp_fp32_pv(const PrefillRunsArgs &a, int h, int kt,
                                            const float (&p)[16], floatx16 (&O)[4]) {
-  const int lane = threadIdx.x & 63, hl = lane >> 5, col = lane & 31;
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));  // addresses are formed here, not ahead of the tile loop
+  const int hl = lane >> 5, col = lane & 31;
   const float *vp = a.v_cache + h * a.kv_stride + (long long)kt * 32 * kHeadDim;  // uniform
   const int last = a.start_pos + a.n_tokens - 1 - kt * 32;
 #pragma unroll
@@ -535,10 +563,9 @@ void prefill_split_kernel(PrefillRunsArgs a) {
 
   half8 qh[8], ql[8];
   floatx16 O[4];
-  float cq, m, l;
+  float unscale_q, m, l;
   int g, g_cap, qrow, q0;
-  bool fp32_q;  // a query of the wave's does not fit pairs (uniform)
-  const float *qp;
+  bool fp32_q;  // a query of the wave's does not fit pairs (uniform): qh and ql hold fp32 values
 
   // Four operands read ahead of the products that use them (two sets of
   // registers in turn): a wave's LDS reads run under its own products.
@@ -586,10 +613,10 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     mm_s(S, L, B, 6);
 #pragma unroll
     for (int r = 0; r < 16; ++r) S[r] = fmaf(L[r], 1.0f / kLowScale, S[r]);
-    float c = fmaxf(cq * exp2i(128 - (wk & 255)), 1e-37f);  // > 0: a masked -inf stays -inf
-    // A marked part's operands are zeros; its products come from the cache.
-    if ((wk & kSplitFp32) || fp32_q) {
-      S = sp_fp32_s(a, h, kt, qp);
+    const float unscale_k = exp2i(128 - (wk & 255));
+    float c = fmaxf(unscale_q * (a.scale_log2 * unscale_k), 1e-37f);  // > 0: a masked -inf stays -inf
+    if (__builtin_expect((wk & kSplitFp32) || fp32_q, 0)) {
+      S = sp_fp32_s(dk, (wk & kSplitFp32) != 0, unscale_k, qh, ql, fp32_q, unscale_q);
       c = a.scale_log2;
     }
     if (kt * 32 + 31 > a.start_pos + q0) {  // the tile reaches the causal diagonal
@@ -612,7 +639,7 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     float t = fmaf(mb, c, -m);
     auto off = [&] { return t + (float)(g - ev - kPMid); };
     const float worst = fmaxf(fmaxf(fabsf(off()), t + (kPHalf - kLazy)), (float)(g - ev - kMaxFactor) + kPHalf);
-    if (zero_v || __ballot(worst > kPHalf) != 0) {
+    if (__builtin_expect(zero_v || __ballot(worst > kPHalf) != 0, 0)) {
       if (t > kLazy) {
         const float mn = ceilf(mb * c);
         const int up = (int)fminf(mn - m, (float)kMaxShift);
@@ -647,8 +674,8 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     }
     l += ls;
     if (zero_v) return;
-    // fp32 products come after these, whose factor is then 0 (a branch around
-    // them would cost 24 more registers than there are)
+    // fp32 products come after these, whose factor is then 0 (a marked part's
+    // operands are zeros; with a branch around them the compiler keeps O twice)
     const float f = fp32_v ? 0.f : ldexpf(1.0f, min(g - ev, kMaxFactor));
     const _Float16 down = (_Float16)(1.0f / kLowScale);
     half8 ph, pl, pq;
@@ -663,7 +690,7 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     pq = ph * down;
     mm_o(A, 0, ph, pl, pq);
     mm_o(B, 2, ph, pl, pq);
-    if (fp32_v) {
+    if (__builtin_expect(fp32_v, 0)) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) p[r] = ldexpf(p[r], g);
       sp_fp32_pv(a, h, kt, p, O);
@@ -679,7 +706,7 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     const int hl = lane >> 5, col = lane & 31;
     q0 = u * UQ + 32 * (wave / G);
     qrow = min(q0 + col, a.n_tokens - 1);
-    qp = a.q + ((long long)qrow * a.n_heads + head) * kHeadDim;
+    const float *qp = a.q + ((long long)qrow * a.n_heads + head) * kHeadDim;
     float4 x[16];
     unsigned mx = 0, en = ~0u;
 #pragma unroll
@@ -696,12 +723,20 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     fp32_q = __ballot(mx != 0 && (no_pairs(mx, en) || (int)(mx >> 23) > kQkTop)) != 0;
     const int e = scale_exp(mx);
     const float sc = exp2i(e);
-    cq = ldexpf(a.scale_log2, -e);
+    unscale_q = ldexpf(1.0f, -e);
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       const float4 v = x[2 * s], w = x[2 * s + 1];
       const float y[8] = {v.x * sc, v.y * sc, v.z * sc, v.w * sc, w.x * sc, w.y * sc, w.z * sc, w.w * sc};
       split8<kLowScale>(y, qh[s], ql[s]);
+    }
+    if (__builtin_expect(fp32_q, 0)) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        qh[s] = *reinterpret_cast<const half8 *>(qp + 16 * s + 8 * hl);
+        ql[s] = *reinterpret_cast<const half8 *>(qp + 16 * s + 8 * hl + 4);
+      }
     }
 #pragma unroll
     for (int db = 0; db < 4; ++db) O[db] = floatx16{};
@@ -786,7 +821,7 @@ void prefill_split_kernel(PrefillRunsArgs a) {
       SP_STAMP(kPfMerged);
     }
     // Lane (col, hl) holds, for r = 4 rq + r3, dims 32 rq + 16 hl + 4 r3 + db.
-    const float inv = 1.0f / (l + __shfl_xor(l, 32));
+    const float inv = 1.0f / sum_half_swap(l);
     if (q0 + col < a.n_tokens) {
       float *op = a.out + ((long long)(q0 + col) * a.n_heads + head) * kHeadDim + 16 * hl;
 #pragma unroll
