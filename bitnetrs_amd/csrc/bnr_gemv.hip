@@ -715,12 +715,12 @@ __global__ __launch_bounds__(256) void lm_head_i8_kernel(LmHeadArgs a) {
 // ---------------------------------------------------------------------------
 // The aligned form on the i8 matrix cores (v_mfma_i32_16x16x64_i8).  The hidden
 // vector becomes fixed point: X[k] = h[k] 2^s with |X| < 2^62, s from the
-// largest |h| (every value within 2^-38 of it keeps its 24 bits, what is cut
-// off is below 2^-61 of it), and X = sum over n < 8 of d[n] 256^n with signed
-// bytes d[n].  A product of 16 rows of weights, as they lie in memory, with the
-// digits as columns sums w d[n] exactly in int32 (2^14 K < 2^31), so the only
-// roundings are those of the eight sums to fp32 and of their scaled total:
-// 4 ulp or so, whatever K (the fp32 sums: 1.7e-7 of the result at K = 2560).
+// largest |h| (every value down to 2^-38 of it keeps its 24 bits), and X = sum
+// over n < 8 of d[n] 256^n with signed bytes d[n].  A product of 16 rows of
+// weights, as they lie in memory, with the digits as columns sums w d[n]
+// exactly in int32 (2^14 K < 2^31), so the only roundings are those of the eight
+// sums to fp32 and of their scaled total: a few 2^-24 of sum |w h|, whatever K
+// (normal data at K = 2560: 4.4e-8 of the result; fp32 sums 1.7e-7).
 //
 // Bound by the weights' stream.  The earlier kernel spent a conversion and an
 // FMA on every weight and read the hidden vector from LDS beside them: 57.3 us
@@ -733,19 +733,57 @@ __global__ __launch_bounds__(256) void lm_head_i8_kernel(LmHeadArgs a) {
 // it).  The pieces change places through 4 KB of LDS per wave, chunk c of row r
 // at slot c ^ r so that neither side has bank conflicts.
 //
-// Infinities and NaN in the hidden vector (no fixed point) take plain fp32
-// sums.
+// A hidden vector that does not fit the fixed point -- an infinity, a NaN, or a
+// nonzero value below 2^-38 of the largest, which would lose bits that count
+// in rows whose weights are zero at the larger ones -- takes fp32 sums
+// (lm_head_fp32_rows).
 // ---------------------------------------------------------------------------
 constexpr int kLmLoads = 8;     // loads of a set: steps of 64 weights of 16 rows
 constexpr int kLmMaxK = 6144;   // digits, 8 bytes per value, beside 16 KB in 64 KB of LDS
 constexpr int kLmWgsPerCu = 4;
+constexpr int kLmRange = 38;    // bits of fixed point below the largest value's significand
 typedef int int4_t __attribute__((ext_vector_type(4)));
+
+// Every row by fp32 products and sums as lm_head_i8_kernel forms them, 16 lanes
+// per row, the whole hidden vector in LDS (s_h: K floats).
+__device__ __forceinline__ void lm_head_fp32_rows(const LmHeadArgs &a, float4 *s_h) {
+  const int tid = threadIdx.x, slot = tid >> 4, j = tid & 15;
+  const int K = a.hidden_size, np = K / 16;
+  for (int g = tid; g < K / 4; g += 256)
+    s_h[(g & 3) * np + (g >> 2)] = *reinterpret_cast<const float4 *>(a.hidden + 4 * g);
+  __syncthreads();
+  for (long long row = (long long)blockIdx.x * 16 + slot; row < a.vocab_size; row += (long long)gridDim.x * 16) {
+    const int8_t *wr = a.weight + row * K;
+    float acc[2] = {0.f, 0.f};
+    constexpr int kAhead = 10;  // loads in flight: a row of 2560 weights
+    for (int c0 = j; c0 < np; c0 += 16 * kAhead) {
+      uint4 w[kAhead];
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        const int c = c0 + 16 * i;
+        w[i] = c < np ? ld16_nt(wr + 16 * c) : make_uint4(0, 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        const int c = c0 + 16 * i;
+        if (c < np) {
+          acc[0] = fma4_i8(w[i].x, s_h[c], acc[0]);
+          acc[1] = fma4_i8(w[i].y, s_h[np + c], acc[1]);
+          acc[0] = fma4_i8(w[i].z, s_h[2 * np + c], acc[0]);
+          acc[1] = fma4_i8(w[i].w, s_h[3 * np + c], acc[1]);
+        }
+      }
+    }
+    const float v = row_sum16_f(acc[0] + acc[1]);
+    if (j == 0) a.out[row] = v * a.scales[row];
+  }
+}
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 void lm_head_mfma_kernel(LmHeadArgs a) {
   extern __shared__ uint4 s_digits[];  // step ks (64 values): digit n's 64 bytes at 512 ks + 64 n
   __shared__ uint4 s_swap[4][256];
-  __shared__ unsigned s_max[4];
+  __shared__ unsigned s_max[4], s_min[4];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int n = lane & 15, u = lane >> 4;
   const int K = a.hidden_size, chunks = (K + 64 * kLmLoads - 1) / (64 * kLmLoads);
@@ -769,28 +807,30 @@ void lm_head_mfma_kernel(LmHeadArgs a) {
 
   // Digits of the hidden vector, four values per thread and round.
   const int quads = chunks * kLmLoads * 16;
-  unsigned mx = 0;
+  // Largest magnitude and one less than the smallest nonzero one (zeros wrap).
+  unsigned mx = 0, mn = ~0u;
   for (int q = tid; 4 * q < K; q += 256) {
     const uint4 h = *reinterpret_cast<const uint4 *>(a.hidden + 4 * q);
-    mx = max(mx, max(max(h.x & 0x7fffffffu, h.y & 0x7fffffffu), max(h.z & 0x7fffffffu, h.w & 0x7fffffffu)));
+    const unsigned b[4] = {h.x & 0x7fffffffu, h.y & 0x7fffffffu, h.z & 0x7fffffffu, h.w & 0x7fffffffu};
+    mx = max(mx, max(max(b[0], b[1]), max(b[2], b[3])));
+    mn = min(mn, min(min(b[0] - 1, b[1] - 1), min(b[2] - 1, b[3] - 1)));
   }
-  for (int m = 1; m < 64; m <<= 1) mx = max(mx, (unsigned)__shfl_xor((int)mx, m));
-  if (lane == 0) s_max[wave] = mx;
+  for (int m = 1; m < 64; m <<= 1) {
+    mx = max(mx, (unsigned)__shfl_xor((int)mx, m));
+    mn = min(mn, (unsigned)__shfl_xor((int)mn, m));
+  }
+  if (lane == 0) {
+    s_max[wave] = mx;
+    s_min[wave] = mn;
+  }
   __syncthreads();
   mx = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
-  if (mx >= 0x7f800000u) {  // uniform over the grid
-    for (; block < blocks; block += stride)
-      for (int r = 0; r < 16; ++r) {
-        const long long row = 16 * block + r;
-        if (row >= a.vocab_size) break;
-        float acc = 0.f;
-        for (int k = lane; k < K; k += 64) acc = fmaf((float)a.weight[row * K + k], a.hidden[k], acc);
-        for (int m = 1; m < 64; m <<= 1) acc += __shfl_xor(acc, m);
-        if (lane == 0) a.out[row] = acc * a.scales[row];
-      }
+  mn = min(min(s_min[0], s_min[1]), min(s_min[2], s_min[3]));
+  const int e_max = max((int)(mx >> 23), 1);
+  if (mx >= 0x7f800000u || max((int)(mn >> 23), 1) < e_max - kLmRange) {  // uniform over the grid
+    lm_head_fp32_rows(a, reinterpret_cast<float4 *>(s_digits));
     return;
   }
-  const int e_max = max((int)(mx >> 23), 1);
   unsigned *digits = reinterpret_cast<unsigned *>(s_digits);
   for (int q = tid; q < quads; q += 256) {
     const uint4 h = 4 * q < K ? *reinterpret_cast<const uint4 *>(a.hidden + 4 * q) : make_uint4(0, 0, 0, 0);
@@ -800,8 +840,8 @@ void lm_head_mfma_kernel(LmHeadArgs a) {
     for (int i = 0; i < 4; ++i) {
       const int ef = (int)(hb[i] >> 23 & 255u);
       const long long m = (long long)((hb[i] & 0x7fffffu) | (ef ? 0x800000u : 0u));
-      const int sh = 38 - (e_max - max(ef, 1));
-      long long x = sh >= 0 ? m << sh : m >> min(-sh, 63);
+      const int sh = kLmRange - (e_max - max(ef, 1));  // >= 0
+      long long x = m << max(sh, 0);  // zeros may lie below the range
       x = (hb[i] >> 31) ? -x : x;
       // signed bytes: add 128 to the lower seven with their carries, then take it off each
       const unsigned long long C = 0x0080808080808080ull;

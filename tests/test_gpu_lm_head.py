@@ -121,6 +121,36 @@ def test_device_lm_head_digits(backend, v, h, kind):
     assert np.all(np.abs(out.cpu().numpy() - exact) <= ulps * 2.0 ** -24 * mag + cut + 1e-44)
 
 
+@pytest.mark.parametrize("h", [48, 2560, 6144])
+@pytest.mark.parametrize("kind", ["above", "below", "both"])
+@pytest.mark.parametrize("e", [31, 38, 39, 45, 60, 100])
+def test_device_lm_head_range(backend, h, kind, e):
+    """One hidden value 2^e above the rest, or a few 2^e below, and rows whose
+    weights see only one side: each row is right to the rounding of its own
+    products, on both sides of what the fixed point holds (2^38)."""
+    case(f"lm head range hidden {h} {kind} 2^{e}")
+    import torch
+
+    v = 300
+    hid, w, sc = workload(v + h + e, v, h)
+    hid = np.where(np.abs(hid) < 0.25, f32(0.5), hid).astype(f32)
+    if kind != "below":
+        hid[5] = 2.0 ** e
+        w[::2, 5] = 0
+    if kind != "above":
+        hid[20:24] *= f32(2.0 ** -e)
+        w[::3] = 0
+        w[::3, 20:24] = 77
+    out = torch.full((v,), float("nan"), device="cuda")
+    backend.dev_lm_head_matmul_i8(torch.from_numpy(hid).cuda(), torch.from_numpy(w.reshape(-1)).cuda(),
+                                  torch.from_numpy(sc).cuda(), out, v, h)
+    torch.cuda.synchronize()
+    exact = (w.astype(np.float64) @ hid.astype(np.float64)) * sc
+    mag = (np.abs(w.astype(np.float64)) @ np.abs(hid).astype(np.float64)) * sc
+    # fp32 sums of 32 chains: h / 32 roundings and a few at the end
+    assert np.all(np.abs(out.cpu().numpy() - exact) <= (h / 32 + 16) * 2.0 ** -24 * mag)
+
+
 def test_device_lm_head_non_finite(backend):
     """An infinity or a NaN in the hidden vector: what fp32 sums give."""
     case("lm head non-finite hidden")
