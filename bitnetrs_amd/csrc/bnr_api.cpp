@@ -301,8 +301,8 @@ struct bnr_ctx {
   int pf_q16 = -1;                // 16-query halves (prefill16_kernel): -1 planner, 0 never, 1 always
   int pf_balanced = -1;           // balanced key chunks: -1 planner, 0 never, 1 always
   // norm-fused GEMV: the most rows per workgroup (16, 32, 64) that keep the
-  // launch at or above this many workgroups
-  int gemv_norm_min_wgs = 128;
+  // launch at or above this many workgroups; 0: by form
+  int gemv_norm_min_wgs = 0;
   int pf_pair = -1;               // paired 16-query launches: -1 planner (4 q heads per kv head), 0 never, 1 where possible
   int pf_split = -1;              // fp16-pair prefill: -1 by shape unless another launch is forced, 0 never, 1 wherever it fits
   std::vector<PrefillPlanEntry> pf_plans;  // recent (shape -> key tiles per chunk) plans
@@ -929,7 +929,7 @@ extern "C" int bnr_create(int device_id, bnr_ctx **out) {
   if (const char *v = std::getenv("BNR_PREFILL_SK_WGS")) c->pf_sk_wgs = std::max(atoi(v), 0);
   if (const char *v = std::getenv("BNR_PREFILL_Q16")) c->pf_q16 = std::min(1, std::max(-1, atoi(v)));
   if (const char *v = std::getenv("BNR_PREFILL_BALANCED")) c->pf_balanced = std::min(1, std::max(-1, atoi(v)));
-  if (const char *v = std::getenv("BNR_GEMV_NORM_MIN_WGS")) c->gemv_norm_min_wgs = std::max(1, atoi(v));
+  if (const char *v = std::getenv("BNR_GEMV_NORM_MIN_WGS")) c->gemv_norm_min_wgs = std::max(0, atoi(v));
   if (const char *v = std::getenv("BNR_PREFILL_PAIR")) c->pf_pair = std::min(1, std::max(-1, atoi(v)));
   if (const char *v = std::getenv("BNR_PREFILL_SPLIT")) c->pf_split = std::min(1, std::max(-1, atoi(v)));
   if (const char *v = std::getenv("BNR_PREFILL_MODE")) {
@@ -2219,15 +2219,23 @@ extern "C" int bnr_dev_ternary_gemv_norm_group(
   g.n = (int)n;
   g.in_features = (int)in_features;
   g.packed_cols = (long long)((in_features + 3) / 4);
-  bool vec = g.packed_cols % 16 == 0;
-  // Rows per workgroup: each workgroup reads all of a (and b) and gamma, so
-  // the launch takes the most rows per workgroup that still leave it
-  // gemv_norm_min_wgs workgroups.
+  // The aligned form also reads the activation vectors as float4 groups.
+  bool vec = g.packed_cols % 16 == 0 && in_features % 16 == 0 && aligned16(a) && aligned16(gamma) &&
+             (mode == BNR_GLUE_PLAIN || aligned16(b)) && (mode != BNR_GLUE_RESIDUAL || aligned16(h_out));
+  for (size_t i = 0; i < n; ++i) vec = vec && aligned16(weight_packed[i]);
+  // Rows per workgroup: each workgroup reads all of a (and b) and gamma, so the
+  // launch takes the most rows per workgroup that still leave it enough
+  // workgroups.  Aligned: 160 (256 CUs; us at least 128 / 160 / 192 / 256
+  // workgroups: 4096 rows, K 6912, 7.9 / 6.1 / 6.0 / 6.1; 8192 rows, K 8192,
+  // 10.6 / 9.1 / 9.1 / 9.1; 5120 rows, K 2560, 4.4 / 4.5 / 4.8 / 4.9; 10240 rows,
+  // K 8192, 10.8 / 10.8 / 12.0 / 12.0).  Element by element, in 256 threads
+  // whatever the rows: 256 (13568 rows, K 2560, 28.1 us with 128, 22.2 with 256).
+  const int min_wgs = c->gemv_norm_min_wgs > 0 ? c->gemv_norm_min_wgs : vec ? 160 : 256;
   int rows = 16;
   for (int r : {64, 32}) {
     long long w = 0;
     for (size_t i = 0; i < n; ++i) w += ((long long)out_features[i] + r - 1) / r;
-    if (w >= c->gemv_norm_min_wgs) {
+    if (w >= min_wgs) {
       rows = r;
       break;
     }
@@ -2245,7 +2253,6 @@ extern "C" int bnr_dev_ternary_gemv_norm_group(
     g.out_features[i] = (int)out_features[i];
     g.wg_off[i] = wgs;
     wgs += (int)((out_features[i] + rows - 1) / rows);
-    vec = vec && ((uintptr_t)weight_packed[i] % 16) == 0;
   }
   for (size_t i = n; i <= (size_t)kMaxGemvGroup; ++i) g.wg_off[i] = wgs;
   if (wgs == 0) return set_ok();
@@ -2257,9 +2264,6 @@ extern "C" int bnr_dev_ternary_gemv_norm_group(
   p.eps = eps;
   p.h_out = mode == BNR_GLUE_RESIDUAL ? h_out : nullptr;
   p.rows = rows;
-  // The vector path also reads the activation vectors as float4 groups.
-  vec = vec && in_features % 16 == 0 && aligned16(a) && aligned16(gamma) &&
-        (mode == BNR_GLUE_PLAIN || aligned16(b)) && (!p.h_out || aligned16(p.h_out));
   DeviceGuard dg(c->device);
   HIP_TRY(launch_ternary_gemv_norm(g, p, vec, (hipStream_t)stream), "ternary_gemv_norm launch");
   return set_ok();

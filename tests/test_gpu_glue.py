@@ -174,6 +174,7 @@ def test_norm_quant_fused(backend, mode, n, alias):
 @pytest.mark.parametrize("k,rows,mode", [(64, (5,), 0), (1024, (40, 7), 1), (1088, (2100,), 0), (3072, (4096, 33), 1),
                                          (3136, (64,), 2), (4096, (130,), 0), (4160, (16,), 1), (6912, (2560,), 2),
                                          (7168, (77,), 0), (7232, (8300,), 2), (8192, (31, 9000), 1), (2560, (6912, 6912), 1),
+                                         (8192, (31, 10240), 2),
                                          (100, (50,), 1), (4200, (20,), 2)])
 def test_gemv_norm_group(backend, k, rows, mode):
     """The norm-fused projection against 64 bits: the residual sum exact; the int8
