@@ -37,10 +37,20 @@ SPLIT_MATRIX_PEAK_TFLOPS = 2500.0 / 3
 
 
 def prefill_peak(n: int, start: int = 0):
-    """(matrix peak, kernel) of a prefill launch: large ones multiply fp16 pairs."""
-    if n >= 512 or n * (start + n // 2) >= 400000:
+    """(matrix peak, kernel) of a prefill launch, by the library's own rule: large
+    ones multiply fp16 pairs.  A launch shape forced by the environment turns
+    that off, unless it forces the pairs."""
+    import ctypes
+
+    from bitnetrs_amd import _lib
+
+    pays = getattr(_lib.load(), "_ZN3bnr18prefill_split_paysEddii")  # bnr::prefill_split_pays
+    pays.restype, pays.argtypes = ctypes.c_bool, [ctypes.c_double, ctypes.c_double, ctypes.c_int, ctypes.c_int]
+    forced = {k: v for k, v in os.environ.items() if k.startswith("BNR_PREFILL_")}
+    split = forced.get("BNR_PREFILL_SPLIT", "-1")
+    if split == "1" or (split == "-1" and set(forced) <= {"BNR_PREFILL_SPLIT"} and pays(n, start, HQ, HKV)):
         return SPLIT_MATRIX_PEAK_TFLOPS, "prefill_split_kernel"
-    return FP32_MATRIX_PEAK_TFLOPS, "prefill16_kernel"
+    return FP32_MATRIX_PEAK_TFLOPS, "fp32 prefill kernels"
 
 
 METRIC = "GQA decode attn GB/s (% HBM peak) @4096 ctx; causal prefill attn TFLOP/s"

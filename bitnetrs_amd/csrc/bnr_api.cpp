@@ -1767,20 +1767,13 @@ long long split_slots(const bnr_ctx *c, long long cap, int n_kv, int group) {
 }
 
 // Whether a prefill of a tiled shape runs as a split launch: nothing else is
-// forced, and (prefill_split_plan, which fills in its runs) its tiles leave at
-// least half of the workspace to the states, and the launch is large enough to
-// pay for the tiles and the longer start: at least kSplitTokens new tokens, or kSplitRows query
-// rows times keys (MI355X, 20/5 heads, RoPE + append + attention in us, fp32
-// launches against split: 256 tokens 18.5 / 22.7, 512 29.9 / 28.6, 1024 62 /
-// 42, 2048 200 / 94, 4000 680 / 267; 64 after 2000 30 / 37, 128 after 3900 59 /
-// 56, 333 after 1207 54 / 43, 512 after 1536 91 / 51).
-constexpr size_t kSplitTokens = 512, kSplitRows = 400000;
-bool prefill_split_shape(const bnr_ctx *c, size_t n_tokens, size_t start_pos) {
+// forced, it pays (prefill_split_pays) and (prefill_split_plan, which fills in
+// its runs) its tiles leave at least half of the workspace to the states.
+bool prefill_split_shape(const bnr_ctx *c, size_t n_tokens, size_t start_pos, size_t n_heads, size_t n_kv) {
   if (c->pf_split >= 0) return c->pf_split != 0;
   const bool forced = c->pf_mode != kPrefillAuto || c->pf_chunk_tiles > 0 || c->pf_q16 >= 0 ||
                       c->pf_balanced >= 0 || c->pf_pair >= 0;
-  return !forced &&
-         (n_tokens >= kSplitTokens || n_tokens * (start_pos + n_tokens / 2) >= kSplitRows);
+  return !forced && prefill_split_pays((double)n_tokens, (double)start_pos, (int)n_heads, (int)n_kv);
 }
 bool prefill_split_plan(const bnr_ctx *c, size_t n_tokens, size_t start_pos, size_t cap,
                         size_t n_heads, size_t n_kv, PrefillRunsArgs &a) {
@@ -1838,7 +1831,7 @@ int prefill_attention_locked(bnr_ctx *c, const float *q, const float *k_cache,
   const long long kv_stride = (long long)(cap * head_dim);
   const int group = (int)(n_heads / n_kv_heads);
   if (prefill_tiled(n_tokens, start_pos, n_heads, n_kv_heads, head_dim, q, k_cache, v_cache, out)) {
-    if (prefill_split_shape(c, n_tokens, start_pos)) {
+    if (prefill_split_shape(c, n_tokens, start_pos, n_heads, n_kv_heads)) {
       PrefillRunsArgs ra{};
       if (prefill_split_plan(c, n_tokens, start_pos, cap, n_heads, n_kv_heads, ra))
         return prefill_split_locked(
@@ -2004,8 +1997,8 @@ extern "C" int bnr_dev_prefill(bnr_ctx *c, float *q, float *k, const float *v, s
   hipStream_t s = (hipStream_t)stream;
   st = ensure_table(c, std::max(start_pos + n_tokens, cap) - 1, head_dim, theta);
   if (st) return st;
-  if (prefill_split_shape(c, n_tokens, start_pos) && aligned16(k) && aligned16(v) &&
-      prefill_tiled(n_tokens, start_pos, n_heads, n_kv_heads, head_dim, q, k_cache, v_cache, out)) {
+  if (prefill_tiled(n_tokens, start_pos, n_heads, n_kv_heads, head_dim, q, k_cache, v_cache, out) &&
+      aligned16(k) && aligned16(v) && prefill_split_shape(c, n_tokens, start_pos, n_heads, n_kv_heads)) {
     PrefillRunsArgs ra{};
     if (prefill_split_plan(c, n_tokens, start_pos, cap, n_heads, n_kv_heads, ra)) {
       st = prefill_split_locked(c, ra,

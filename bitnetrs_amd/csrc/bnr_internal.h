@@ -581,6 +581,8 @@ static_assert(sizeof(PrefillRunsArgs) <= 4096, "PrefillRunsArgs exceeds the kern
 // n_kv for workgroups of `group` heads on n_cu CUs, with at most max_slots
 // states per kv head.  False when the shape does not fit the words.
 bool plan_prefill_runs(PrefillRunsArgs &a, int group, int n_cu, long long max_slots);
+// Whether a split launch of this shape is expected to beat the fp32 launches.
+bool prefill_split_pays(double n_tokens, double start_pos, int n_heads, int n_kv);
 hipError_t launch_prefill_split(const PrefillRunsArgs &a, int group, hipStream_t s);
 // Stream-K prefill over `wgs` workgroups (a.sk_units, a.sk_per_head set by
 // prefill_streamk_units).

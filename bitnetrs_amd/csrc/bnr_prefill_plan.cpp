@@ -629,6 +629,28 @@ bool plan_prefill_runs(PrefillRunsArgs &a, int group, int n_cu, long long max_sl
   return true;
 }
 
+// The fp32 launches take their products' time and a share that grows more
+// slowly with the cached rows; the split ones save most of the first, but write
+// every row's tile before they start, and their starts and piece ends are
+// longer.  Over 1956 shapes (16 to 1536 tokens after 0 to 32000 rows; 2, 4 and 8
+// query heads on 1 to 10 kv heads; RoPE + append + attention replayed in HIP
+// graphs, MI355X, 256 CUs) the two take the same time where query rows x keys
+// is about a constant times the square root of the keys.  With 4 query heads the
+// constant grows with the kv heads up to 5, and the tiles show as 25 per cached
+// row.  With this line the launch taken is 0.6 % above the better one on
+// average (with "512 tokens or 400000 tokens x keys" 2.3 %).  us, fp32 / split:
+// 20/5 heads: 512 tokens 30.4 / 30.3, 1024 61.6 / 43.0; 128 after 2000 38.9 /
+// 40.8, 256 after 2000 61.7 / 50.4; 64 after 8000 67.6 / 61.6; 16 after 32000 103
+// / 140.  4/1: 512 25.4 / 25.7.  2/1: 512 18.8 / 24.4, 1536 32.2 / 32.7.  16/2:
+// 512 34.0 / 37.2, 768 47.2 / 40.5.
+bool prefill_split_pays(double n_tokens, double start_pos, int n_heads, int n_kv) {
+  const int group = n_heads / n_kv;
+  const double rows = start_pos + n_tokens, pairs = n_heads * n_tokens * (start_pos + 0.5 * n_tokens);
+  if (group > 4) return pairs >= 130e3 * std::sqrt(rows);
+  if (group > 2) return pairs >= 26e3 * std::min(n_kv, 5) * std::sqrt(rows) + 25.0 * n_kv * rows;
+  return pairs >= 44e3 * std::min(n_kv, 2) * std::sqrt(rows);
+}
+
 // (kv head, item) pairs a planned chunked launch may use on a cache of cap
 // rows: four chunks per query tile on average over the cap/32 query tiles,
 // and never more than kPrefillMaxPlannedItems.  Replaying the planner over

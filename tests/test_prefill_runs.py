@@ -1,6 +1,7 @@
 """The runs of split prefill launches (bnr::plan_prefill_runs): a host-only
 harness built against the library decodes every run of 4000 seeded plans the
-way the kernel does (no GPU needed)."""
+way the kernel does, and checks on which side of the line between split and
+fp32 launches measured shapes fall (no GPU needed)."""
 import os
 import shutil
 import subprocess
