@@ -494,17 +494,20 @@ __device__ __forceinline__ void sp_fp32_pv(const PrefillRunsArgs &a, int h, int 
 // flight, does not wait for them there: prefill_split_kernel waits for its
 // copies itself, before the barrier that opens the buffer.  The copies have no
 // register results, and a wait the compiler places for its own loads only
-// becomes stricter by them.  (m0 is reserved: nothing else in this file's
-// kernels uses it.)
+// becomes stricter by them.  m0, which the
+// compiler does not let an asm declare as changed, is put back.
 __device__ __forceinline__ void dma4k(const char *src, unsigned lane16, unsigned lds) {
+  unsigned m0;
   asm volatile(
-      "s_mov_b32 m0, %0\n\t"
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %1\n\t"
       "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, %2\n\t"
-      "global_load_lds_dwordx4 %1, %2 offset:1024\n\t"
-      "global_load_lds_dwordx4 %1, %2 offset:2048\n\t"
-      "global_load_lds_dwordx4 %1, %2 offset:3072"
-      :
+      "global_load_lds_dwordx4 %2, %3\n\t"
+      "global_load_lds_dwordx4 %2, %3 offset:1024\n\t"
+      "global_load_lds_dwordx4 %2, %3 offset:2048\n\t"
+      "global_load_lds_dwordx4 %2, %3 offset:3072\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(m0)
       : "s"(lds), "v"(lane16), "s"(src)
       : "memory");
 }
