@@ -222,15 +222,17 @@ __global__ __launch_bounds__(256) void ternary_gemv_group_kernel(TernaryGemvGrou
 // ---------------------------------------------------------------------------
 // Ternary GEMV with the activation's RMSNorm and int8 quantisation as its
 // prologue (the glue launch folded into the projection).  Every workgroup
-// forms x from f32 inputs (a | a + b | max(a,0)^2 * b), reduces sum(x^2) and
-// max|y| with the same tree, and so derives the same int8 activations and
-// the same scale as norm_quant_kernel would; the int8 vector never leaves
-// LDS.  The aligned kernel below issues the (cache-resident) activation loads
+// forms x from f32 inputs (a | a + b | max(a,0)^2 * b) and reduces sum(x^2) and
+// max|y| with one tree, so that a launch's workgroups agree on every int8
+// activation and on the scale; the int8 vector never leaves LDS.  The order of
+// the sum is not norm_quant_kernel's, and differs between the forms here (quads
+// over 256 or 512 threads, 16 consecutive values per thread): y agrees to
+// rounding, and an activation at a half-way case may differ by one.  The aligned kernel below issues the (cache-resident) activation loads
 // first and its weight loads right after, so the prologue runs under the
 // weights' latency; the one here takes unaligned rows and vectors and any K <=
 // 4096 NG (NG = 1 or 2 16-activation groups per thread), element by element.
 // Workgroup 0 writes h_out (mode residual), which must not alias a or b.
-// A workgroup owns 256 / LPR rows, LPR lanes per row: every workgroup reads
+// A workgroup of T threads owns T / LPR rows, LPR lanes per row: every workgroup reads
 // the whole of a (and b) and gamma, so a launch with many rows takes 32 or
 // 64 rows per workgroup to read those vectors fewer times.
 // ---------------------------------------------------------------------------
