@@ -90,10 +90,11 @@ def test_lm_head_shape_errors_match_oracle(backend):
 def test_device_lm_head_digits(backend, v, h, kind):
     """The i8 matrix-core form at its edges -- one row, part of a block, several
     blocks per wave, K within and past a set of loads, its largest K and the
-    form beyond it -- and over magnitudes: values 2^-40 to 1, one value 2^30
-    times the others (and zero weights there, so that the rest must survive),
-    subnormals, zeros.  fp32 sums would be off by up to K ulp of the products'
-    magnitude; eight exact sums rounded once are off by a few."""
+    form beyond it -- and over magnitudes: values 2^-40 to 1 (past what fixed
+    point holds: fp32 sums), one value 2^30 times the others (and zero weights
+    there, so that the rest must survive), subnormals, zeros.  fp32 sums may be
+    off by up to K ulp of the products' magnitude; eight exact sums rounded once
+    are off by a few."""
     case(f"lm head digits vocab {v} hidden {h} {kind}")
     import torch
 
