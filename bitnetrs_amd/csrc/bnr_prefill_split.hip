@@ -111,6 +111,9 @@ __device__ __forceinline__ void mag4(float4 x, unsigned &mx, unsigned &elem_min)
   mx = max(mx, max(max(b[0], b[1]), max(b[2], b[3])));
   elem_min = min(elem_min, min(min(b[0] - 1, b[1] - 1), min(b[2] - 1, b[3] - 1)));
 }
+__device__ __forceinline__ unsigned least4(float4 x) {
+  return min(min(abs_bits(x.x), abs_bits(x.y)), min(abs_bits(x.z), abs_bits(x.w)));
+}
 __device__ __forceinline__ float exp2i(int e) {  // 2^e, -126 <= e <= 127
   return __builtin_bit_cast(float, (unsigned)(e + 127) << 23);
 }
@@ -163,12 +166,18 @@ __device__ __forceinline__ int v_word(unsigned mx, unsigned row_min, unsigned el
 }
 // A K tile's.  Values past 2^54 are marked: the scales of K and q and their
 // product then stay inside fp32 (a score may be small all the same, where K
-// or q has zeros).
-constexpr int kQkTop = 127 + 54;
-__device__ __forceinline__ int k_word(unsigned mx, unsigned elem_min) {
-  if (mx == 0) return 128 | kSplitZero;
-  const bool fp32 = no_pairs(mx, elem_min) || (int)(mx >> 23) > kQkTop;
-  return (scale_exp(mx) + 128) | (fp32 ? kSplitFp32 : 0);
+// or q has zeros).  kSplitWide: a zero, or a value below 2^-24 of the largest
+// (least: the smallest magnitude).  In a tile without, a key's values are within
+// 2^24 of one another, and what a q pair cuts off, 2^-51 of the row's largest
+// value, is 2^-27 at most of what that largest value adds to the score.
+constexpr int kQkTop = 127 + 54, kWideRange = 24;
+constexpr int kSplitWide = 0x400, kSplitAny = 0x800;  // kSplitAny: in every K word
+__device__ __forceinline__ int k_word(unsigned mx, unsigned elem_min, unsigned least) {
+  if (mx == 0) return 128 | kSplitZero | kSplitAny;
+  const int e = (int)(mx >> 23);
+  const bool fp32 = no_pairs(mx, elem_min) || e > kQkTop;
+  const bool wide = (int)(least >> 23) < max(1, e - kWideRange);
+  return (scale_exp(mx) + 128) | (fp32 ? kSplitFp32 : 0) | (wide ? kSplitWide : 0) | kSplitAny;
 }
 // The scale exponent that a V tile asks of O.  A marked tile's values are not
 // scaled: the limits keep its weights, 2^(15 + exponent) at most, and their
@@ -230,7 +239,7 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
     }
     return;
   }
-  __shared__ unsigned s_vmax[2], s_vmin[2], s_velem[2], s_kmax[2], s_kelem[2];
+  __shared__ unsigned s_vmax[2], s_vmin[2], s_velem[2], s_kmax[2], s_kelem[2], s_kleast[2];
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int hl = lane >> 5, col = lane & 31;
   const int h = (int)blockIdx.x % a.n_kv, kt = (int)blockIdx.x / a.n_kv;
@@ -333,22 +342,25 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
       }
     }
   }
-  unsigned mx = 0, en = ~0u;
+  unsigned mx = 0, en = ~0u, least = ~0u;
 #pragma unroll
   for (int u = 0; u < 2; ++u)
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
       mag4(lo[u][e], mx, en);
       mag4(hi[u][e], mx, en);
+      least = min(least, min(least4(lo[u][e]), least4(hi[u][e])));
     }
   mx = wave_red<true>(mx);
   en = wave_red<false>(en);
+  least = wave_red<false>(valid ? least : ~0u);
   if (lane == 0) {
     s_kmax[w] = mx;
     s_kelem[w] = en;
+    s_kleast[w] = least;
   }
   __syncthreads();
-  const int word = k_word(max(s_kmax[0], s_kmax[1]), min(s_kelem[0], s_kelem[1]));
+  const int word = k_word(max(s_kmax[0], s_kmax[1]), min(s_kelem[0], s_kelem[1]), min(s_kleast[0], s_kleast[1]));
   const bool marked = (word & kSplitFp32) != 0;
   const float sc = exp2i((word & 255) - 128);
   if (tid == 128) info->x = word;
@@ -431,6 +443,13 @@ __device__ __forceinline__ float sum_half_swap(float v) {
   return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
 }
 
+// The lane, formed where it is used and not kept.
+__device__ __forceinline__ int lane_here() {
+  int lane;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(lane));
+  return lane;
+}
+
 __device__ __forceinline__ half8 ld_op(const float *lds, int op) {
   return *reinterpret_cast<const half8 *>(lds + op * 256 + 4 * (threadIdx.x & 63));
 }
@@ -444,11 +463,12 @@ __device__ __forceinline__ float op_value(half8 x, half8 y, int i, bool fp32, fl
 }
 
 // S^T of a tile with fp32 products (v_mfma_f32_32x32x2_f32): step 8 s + i takes
-// dim 16 s + 8 (lane / 32) + i.  K and q each as pairs (unscale_k, unscale_q
-// undo their scales) or fp32 values.  The caller's scale is log2(e) / sqrt(d)
-// alone.
+// dim 16 s + 8 (lane / 32) + i.  K as pairs (unscale_k undoes their scale) or
+// fp32 values; q as pairs or, where they have lost bits, read from memory (qp:
+// the lane's values of step 0, or null).  The caller's scale is log2(e) /
+// sqrt(d) alone.
 __device__ __forceinline__ floatx16 sp_fp32_s(const float *dk, bool fp32_k, float unscale_k, const half8 (&qh)[8],
-                                              const half8 (&ql)[8], bool fp32_q, float unscale_q) {
+                                              const half8 (&ql)[8], float unscale_q, bool q_lost, const float *qp) {
   floatx16 S = floatx16{};
   // hidden from the compiler, which would otherwise form q's 64 values ahead of
   // the tile loop and keep them in registers
@@ -457,10 +477,15 @@ __device__ __forceinline__ floatx16 sp_fp32_s(const float *dk, bool fp32_k, floa
   for (int s = 0; s < 8; ++s) {
     __builtin_amdgcn_sched_barrier(0);
     const half8 x = ld_op(dk, 2 * s), y = ld_op(dk, 2 * s + 1);
+    half8 u = qh[s], v = ql[s];
+    if (q_lost) {
+      u = *reinterpret_cast<const half8 *>(qp + 16 * s);
+      v = *reinterpret_cast<const half8 *>(qp + 16 * s + 4);
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       S = __builtin_amdgcn_mfma_f32_32x32x2f32(op_value(x, y, i, fp32_k, unscale_k),
-                                               op_value(qh[s], ql[s], i, fp32_q, unscale_q), S, 0, 0, 0);
+                                               op_value(u, v, i, q_lost, unscale_q), S, 0, 0, 0);
   }
   __builtin_amdgcn_sched_barrier(0);
   return S;
@@ -568,7 +593,8 @@ void prefill_split_kernel(PrefillRunsArgs a) {
   floatx16 O[4];
   float unscale_q, m, l;
   int g, g_cap, qrow, q0;
-  bool fp32_q;  // a query of the wave's does not fit pairs (uniform): qh and ql hold fp32 values
+  int q_words;  // bits of the K words whose tiles take fp32 scores (uniform): kSplitFp32, and more where
+                // a query of the wave's has lost bits as a pair
 
   // Four operands read ahead of the products that use them (two sets of
   // registers in turn): a wave's LDS reads run under its own products.
@@ -618,8 +644,10 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     for (int r = 0; r < 16; ++r) S[r] = fmaf(L[r], 1.0f / kLowScale, S[r]);
     const float unscale_k = exp2i(128 - (wk & 255));
     float c = fmaxf(unscale_q * (a.scale_log2 * unscale_k), 1e-37f);  // > 0: a masked -inf stays -inf
-    if (__builtin_expect((wk & kSplitFp32) || fp32_q, 0)) {
-      S = sp_fp32_s(dk, (wk & kSplitFp32) != 0, unscale_k, qh, ql, fp32_q, unscale_q);
+    if (__builtin_expect((wk & q_words) != 0, 0)) {
+      const int lane = lane_here(), row = min(q0 + (lane & 31), a.n_tokens - 1);
+      const float *qp = a.q + ((long long)row * a.n_heads + head) * kHeadDim + 8 * (lane >> 5);
+      S = sp_fp32_s(dk, (wk & kSplitFp32) != 0, unscale_k, qh, ql, unscale_q, q_words != kSplitFp32, qp);
       c = a.scale_log2;
     }
     if (kt * 32 + 31 > a.start_pos + q0) {  // the tile reaches the causal diagonal
@@ -701,8 +729,7 @@ void prefill_split_kernel(PrefillRunsArgs a) {
   };
 
   // Queries of the unit's block: lane's dims 16 s + 8 hl + i of query q0 + col
-  // (rows past the end repeat the last and are not stored), as fp16 pairs.  A
-  // query that does not fit them takes its wave through fp32 scores.
+  // (rows past the end repeat the last and are not stored), as fp16 pairs.
   auto begin = [&] {
     int lane = tid & 63;
     asm volatile("" : "+v"(lane));
@@ -723,7 +750,13 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     mx = max((unsigned)r[0], (unsigned)r[1]);
     const auto re = __builtin_amdgcn_permlane32_swap(en, en, false, false);
     en = min((unsigned)re[0], (unsigned)re[1]);
-    fp32_q = __ballot(mx != 0 && (no_pairs(mx, en) || (int)(mx >> 23) > kQkTop)) != 0;
+    // Values below 2^-28 of the row's largest have lost bits, which counts with
+    // some K tiles; an infinity, a NaN or a value past 2^54 with all.  (A small
+    // row has nothing to lose: its scores with K up to 2^54 are.)
+    const int e_mx = (int)(mx >> 23);
+    q_words = kSplitFp32;
+    if (__ballot((int)(en >> 23) < max(1, e_mx - kElemRange)) != 0) q_words |= kSplitWide;
+    if (__ballot(e_mx > kQkTop) != 0) q_words |= kSplitAny;
     const int e = scale_exp(mx);
     const float sc = exp2i(e);
     unscale_q = ldexpf(1.0f, -e);
@@ -732,14 +765,6 @@ void prefill_split_kernel(PrefillRunsArgs a) {
       const float4 v = x[2 * s], w = x[2 * s + 1];
       const float y[8] = {v.x * sc, v.y * sc, v.z * sc, v.w * sc, w.x * sc, w.y * sc, w.z * sc, w.w * sc};
       split8<kLowScale>(y, qh[s], ql[s]);
-    }
-    if (__builtin_expect(fp32_q, 0)) {
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        qh[s] = *reinterpret_cast<const half8 *>(qp + 16 * s + 8 * hl);
-        ql[s] = *reinterpret_cast<const half8 *>(qp + 16 * s + 8 * hl + 4);
-      }
     }
 #pragma unroll
     for (int db = 0; db < 4; ++db) O[db] = floatx16{};
