@@ -665,12 +665,22 @@ void prefill_split_kernel(PrefillRunsArgs a) {
     const bool zero_v = (wv & kSplitZero) != 0;
     bool fp32_v = (wv & kSplitFp32) != 0;
     // t: log2 of the tile's largest weight; off: of its largest operand, past
-    // the middle of the range.  One comparison for "t > kLazy, |off| > kPHalf
-    // or a factor too large".
+    // the middle of the range.  One comparison for "t > kLazy, |off| > kPHalf, a
+    // factor too large or a score of 2^22 and more".
     float t = fmaf(mb, c, -m);
     auto off = [&] { return t + (float)(g - ev - kPMid); };
-    const float worst = fmaxf(fmaxf(fabsf(off()), t + (kPHalf - kLazy)), (float)(g - ev - kMaxFactor) + kPHalf);
+    const float worst = fmaxf(fmaxf(fmaxf(fabsf(off()), t + (kPHalf - kLazy)), (float)(g - ev - kMaxFactor) + kPHalf),
+                              fabsf(mb * c) * (kPHalf * 0x1p-22f));
     if (__builtin_expect(zero_v || __ballot(worst > kPHalf) != 0, 0)) {
+      if (__ballot(fabsf(mb * c) > 0x1p22f && mb > -INFINITY) != 0) {
+        // S c rounded once, in m and in the weights alike: what a fused product
+        // keeps of it could be more than the weights' range here
+#pragma unroll
+        for (int r = 0; r < 16; ++r) S[r] *= c;
+        mb *= c;
+        c = 1.0f;
+        t = mb - m;
+      }
       if (t > kLazy) {
         const float mn = ceilf(mb * c);
         const int up = (int)fminf(mn - m, (float)kMaxShift);

@@ -200,17 +200,22 @@ def test_k_apart(monkeypatch, other, r):
     check(monkeypatch, q, kc, vc, start)
 
 
-# q: one head dim far above the rest, K zero or as far below the rest there; in
-# every row or in a few
+# q: one head dim far above the rest, K zero, as far below the rest or 2^-24 of
+# the rest there (the line up to which tiles take q's pairs whatever they lost);
+# in every row or in a few
 @pytest.mark.parametrize("r", RATIOS)
-@pytest.mark.parametrize("other", ["zero", "inverse"])
+@pytest.mark.parametrize("other", ["zero", "inverse", "line"])
 @pytest.mark.parametrize("every", [1, 50])
 def test_q_apart(monkeypatch, other, every, r):
     case(f"split prefill, a q dim of {r} in every {every} rows, K {other}")
     n, start = 544, 64
     q, kc, vc = normal(n, start, 16)
     q.view(n, HQ, D)[::every, :, 5] *= r
-    kc[:, :, 5] *= 0.0 if other == "zero" else 1 / r
+    kc[:, :, 5] *= {"zero": 0.0, "inverse": 1 / r, "line": max(1 / r, 2.0 ** -24)}[other]
+    if other == "line":  # no value of a tile below 2^-24 of its largest
+        import torch
+
+        kc[:] = torch.where(kc.abs() < 0.25 * kc.abs().amax(dim=1, keepdim=True), 0.25 * kc.abs().amax(dim=1, keepdim=True), kc)
     check(monkeypatch, q, kc, vc, start)
 
 
