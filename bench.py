@@ -1463,8 +1463,8 @@ def main() -> int:
             "value": round(lm["gbs"], 2), "unit": "GB/s", "us_per_token": round(lm["us"], 3),
             "roofline": {"bound": "hbm", "achieved": round(lm["gbs"], 2), "peak": HBM_PEAK_GBS,
                          "unit": "GB/s", "frac": round(lm["gbs"] / HBM_PEAK_GBS, 4),
-                         "traffic": traffic.get("lm_head_i8_kernel", {}).get("bytes_per_launch"),
-                         "kernel": "lm_head_i8_kernel", "kernel_us": round(lm["us"], 3),
+                         "traffic": traffic.get("lm_head_mfma_kernel", {}).get("bytes_per_launch"),
+                         "kernel": "lm_head_mfma_kernel", "kernel_us": round(lm["us"], 3),
                          "bytes_per_launch": lm["bytes"]}}
     if not args.no_model:
         md = bench_model(torch, be)
