@@ -8,15 +8,18 @@
 // at 3/16 of its matrix-core time.  The sums are shorter as well: a 32 x 32 x
 // 16 product adds 16 terms before it rounds, the fp32 one 2.  Measured
 // against 64 bits the outputs are closer than the fp32 kernels' (relative
-// 2-norm, fp32 products -> pairs: 1024 tokens 3.7 -> 2.9e-7, 2048 3.8 -> 3.2e-7,
-// 333 after 1207 5.3 -> 4.0e-7).
+// 2-norm, fp32 products -> pairs: 1024 tokens 3.7 -> 2.0e-7, 2048 3.8 -> 2.4e-7,
+// 333 after 1207 5.3 -> 2.8e-7).
 //
 // The scales 2^e are exact powers of two that put the largest magnitude of a
-// 32-key tile of K, of V, or of a query row in [2^14, 2^15): what the fp16
-// subnormals cut off is then 2^-39 of that largest magnitude.  A tile that
-// holds an infinity or a NaN, or rows so far apart that the smallest one
-// would lose bits (kSplitRange), is marked, and the attention kernel takes
-// it with fp32 products from the cache (its operands are then zeros).
+// 32-key tile of K, of V, or of a query row in [2^14, 2^15), and l is stored
+// times 2^12 (kLowScale): values down to 2^-28 of that largest one keep their
+// bits.  A K or V tile with a nonzero value below that, an infinity, a NaN, or
+// (V) rows far apart is marked and takes fp32 products, which the attention
+// kernel has beside the others; so does a query row, against the K tiles where
+// what it lost counts.  One K or V tile in 20000 of normal data is marked.  With
+// one K and one V dim 2^30 above the others in every row all are: 2048 tokens
+// then take 311 us (K alone 202, V alone 184; the fp32 launches 186).
 //
 //   prefill_split_kv_kernel  K/V tiles -> fp16 pairs in MFMA operand order
 //                            (with RoPE of q/k and the append fused in)
@@ -392,19 +395,22 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
 // Register r of a 32 x 32 accumulator holds row 8 (r / 4) + 4 (lane / 32) +
 // r % 4; row i of O^T's dim block db is head dim 4 i + db.
 //
-// Two workgroups share a CU (232 registers, 64 KB of LDS): one's softmax,
+// Two workgroups share a CU (218 registers, 64 KB of LDS): one's softmax,
 // starts and ends run under the other's products.  A workgroup's waves share a
 // tile's operands; the next tile's go to the other LDS buffer while this one
 // is multiplied, one barrier per tile.  One round: every CU gets two runs of
 // about equal cost, and no item list is decoded.
 //
-// A tile of 32 queries x 4 heads takes 0.83 us of matrix-core time per CU (at
-// the 1.85 GHz this load runs at) and 1.2 - 1.5 us as measured with two
-// workgroups: the younger one's products wait for the older's, and what is
-// left of it then runs alone.  With RoPE and append (20/5 heads, MI355X):
-// 1024 tokens 60 -> 40 us, 2048 199 -> 90, 333 after 1207 53 -> 42 against the
-// fp32 products.  One 8-wave workgroup of 64 queries per CU (half the
-// operand traffic, one barrier per 64 keys) took 47, 93 and 48 us.
+// A tile of 32 queries x 4 heads takes 1536 cycles of a SIMD's matrix core (0.7
+// us at the 2.2 GHz that the counters read) and 1.15 us per CU as measured with
+// two workgroups (each 2.3): the younger one's products wait for the older's,
+// and what is left of it then runs alone.  At 2048 tokens the matrix cores are
+// busy 38 % of the cycles, at 1024 (5 tiles a run) 18 %: starts 5 us, a piece's
+// end 4 to 6.  No LDS bank conflicts.  With RoPE and append (20/5 heads,
+// MI355X): 1024 tokens 60 -> 40 us, 2048 199 -> 89, 333 after 1207 53 -> 42
+// against the fp32 products.  One 8-wave workgroup of 64 queries per CU (half
+// the operand traffic, one barrier per 64 keys) took 47, 93 and 48 us (before
+// low halves were scaled).
 //
 // p = exp2(S c - m): c undoes the scales of K and q and applies log2(e) /
 // sqrt(d); m is a lazily moved whole number above or near the query's largest
@@ -414,8 +420,9 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
 // O holds sum(p V) 2^g, g a whole number per query, and the operand is p
 // 2^(g - ev) for a V tile of scale exponent ev.  g stays while the tile's
 // largest operand lies between 2^1 (what fp16's subnormals cut off is then 2^-26
-// of it) and 2^15, else it is moved to 2^8, and O with it.  Weights and
-// V so far below what O holds that it would overflow (kScaleSpan), and weights
+// of it) and 2^15, else it is moved to 2^8, and O with it (scores of 4 times the
+// spread of normal data move it in most tiles: 2048 tokens 97 us for 91).
+// Weights and V so far below what O holds that it would overflow (kScaleSpan), and weights
 // near fp32's end, take fp32 products for that tile.  The output is (O / l)
 // 2^-g in that order: O alone, with the sum of the weights and a power of two in
 // it, would pass fp32's largest value where the output does not.
@@ -424,8 +431,8 @@ __global__ __launch_bounds__(256) void prefill_split_kv_kernel(PrefillSplitArgs 
 #pragma clang diagnostic ignored "-Wpass-failed"
 
 constexpr float kLazy = 4.0f, kNoRef = -3.4028234e38f, kLeastP = -126.0f, kPHalf = 7.0f;
-constexpr int kPMid = 8;           // operands: the tile's largest is 2^8, in 2^(8 -+ 7)
-constexpr int kScaleSpan = 72;     // sum(p V) 2^g <= 2^23 times the keys, and 2^72 more once g follows V down
+constexpr int kPMid = 8;            // operands: the tile's largest is 2^8, in 2^(8 -+ 7)
+constexpr int kScaleSpan = 72;      // sum(p V) 2^g <= 2^23 times the keys, and 2^72 more once g follows V down
 constexpr int kNoScale = 1 << 28;   // O holds nothing yet
 constexpr int kMaxFactor = 112;     // of 2^(g - ev), a float
 constexpr int kMaxShift = 4096;     // more than any O keeps
