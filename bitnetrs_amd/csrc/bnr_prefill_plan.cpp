@@ -636,7 +636,7 @@ bool plan_prefill_runs(PrefillRunsArgs &a, int group, int n_cu, long long max_sl
 // query heads on 1 to 10 kv heads; RoPE + append + attention replayed in HIP
 // graphs, MI355X, 256 CUs) the two take the same time where query rows x keys
 // is about a constant times the square root of the keys.  With 4 query heads the
-// constant grows with the kv heads up to 5, and the tiles show as 25 per cached
+// constant grows with the kv heads up to 5, and the tiles show as 40 per cached
 // row.  With this line the launch taken is 0.6 % above the better one on
 // average (with "512 tokens or 400000 tokens x keys" 2.3 %).  us, fp32 / split:
 // 20/5 heads: 512 tokens 30.4 / 30.3, 1024 61.6 / 43.0; 128 after 2000 38.9 /
@@ -647,7 +647,7 @@ bool prefill_split_pays(double n_tokens, double start_pos, int n_heads, int n_kv
   const int group = n_heads / n_kv;
   const double rows = start_pos + n_tokens, pairs = n_heads * n_tokens * (start_pos + 0.5 * n_tokens);
   if (group > 4) return pairs >= 130e3 * std::sqrt(rows);
-  if (group > 2) return pairs >= 26e3 * std::min(n_kv, 5) * std::sqrt(rows) + 25.0 * n_kv * rows;
+  if (group > 2) return pairs >= 22.5e3 * std::min(n_kv, 5) * std::sqrt(rows) + 40.0 * n_kv * rows;
   return pairs >= 44e3 * std::min(n_kv, 2) * std::sqrt(rows);
 }
 
