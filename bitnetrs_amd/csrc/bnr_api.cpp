@@ -1806,7 +1806,6 @@ int prefill_split_locked(bnr_ctx *c, PrefillRunsArgs &pa, const RopeAppendArgs &
   sa.info = reinterpret_cast<int2 *>(c->pf_ws + n_kv * sa.tiles_per_head * kSplitTileFloats);
   HIP_TRY(launch_prefill_split_kv(sa, s), "prefill tiles launch");
   pa.q = rope_args.q;
-  pa.k_cache = rope_args.k_cache;
   pa.v_cache = rope_args.v_cache;
   pa.kv_stride = rope_args.kv_stride;
   pa.out = out;

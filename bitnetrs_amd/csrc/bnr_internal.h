@@ -557,7 +557,7 @@ constexpr int kSplitStateFloats = 68 * 64;  // a wave's state: O, and (m, l, g, 
 constexpr int kMaxPrefillRuns = 256;
 struct PrefillRunsArgs {
   const float *q;                  // [n_tokens][n_heads][128], rotated
-  const float *k_cache, *v_cache;  // [n_kv][cap][128] (marked tiles)
+  const float *v_cache;            // [n_kv][cap][128] (marked tiles)
   long long kv_stride;
   float *out;                      // [n_tokens][n_heads][128]
   int n_tokens, start_pos, n_heads, n_kv;
